@@ -15,33 +15,18 @@
 // same bits). 16-bit outputs leave through LDS as 16-byte row pieces.
 //
 // attn_f32_mfma (fp32 inputs, head_dim 32 or 64, 16-byte aligned rows): fp32 matrix cores for both products, the key
-// range split over the 4 waves of a 32-query workgroup; the reference's float attention surface at fp32 accuracy.
+// range split over the 4 waves of a 32-query workgroup; the reference's float attention surface at fp32 accuracy. For
+// few keys, and calls without the workspace attn_f32_split (attention_f32.hip) cuts its key range into.
 //
 // attn_f32 (any dtype, head_dim <= 256): one wave per (query, head, batch), 64 keys per step with one key per lane
 // for the scores and the head dimension split over lanes for P * V; fp32 throughout. Used for the remaining fp32
 // cases (unaligned rows, other head sizes) and 16-bit inputs with head sizes other than 64.
-#include "common.h"
+#include "attention.h"
 
 #include <type_traits>
 
 namespace idolq {
 namespace {
-
-struct AttnParams {
-    const void* q;
-    const void* k;
-    const void* v;
-    void* out;
-    int dt, out_dt;
-    int64_t lq, lk, heads, head_dim;
-    int64_t ldq, ldkv, q_bs, kv_bs, ldo, o_bs;
-    float scale_log2;  // log2(e) / sqrt(head_dim)
-    // V staged ahead of attn_mfma_hd64<bf16, true> by attn_v_tiles: fp16 V^T tiles and their exponents
-    const uint16_t* vt;
-    const int* vexps;
-    int64_t ntiles;
-    int out_vec;  // out has the input dtype and 16-byte aligned rows and batches: rows go out as 16-byte stores
-};
 
 constexpr int kHD = 64;
 constexpr int kBQ = 128;
@@ -737,6 +722,9 @@ __global__ __launch_bounds__(256) void attn_f32_mfma(AttnParams p) {
 using namespace idolq;
 
 namespace {
+// fp32 calls the matrix-core kernels take (with 16-byte aligned rows)
+bool f32_matrix(int dtype, int64_t head_dim) { return dtype == IDOLQ_F32 && (head_dim == 32 || head_dim == 64); }
+
 // The staged V^T tiles and their exponents of a bf16 call with head_dim 64 (0 bytes for any other call).
 size_t attn_workspace_bytes(int dtype, int64_t batch, int64_t lk, int64_t heads, int64_t head_dim) {
     if (dtype != IDOLQ_BF16 || head_dim != kHD || batch <= 0 || lk <= 0 || heads <= 0) return 0;
@@ -744,6 +732,11 @@ size_t attn_workspace_bytes(int dtype, int64_t batch, int64_t lk, int64_t heads,
     return tiles * kHD * kBKV * 2 + (tiles * 4 + 255) / 256 * 256;
 }
 }  // namespace
+
+extern "C" size_t idolq_attention_f32_workspace(int64_t batch, int64_t lq, int64_t lk, int64_t heads, int64_t head_dim) {
+    if (batch <= 0 || lq <= 0 || lk <= 0 || heads <= 0 || !f32_matrix(IDOLQ_F32, head_dim)) return 0;
+    return attn_f32_workspace_bytes(batch, lq, heads, head_dim, attn_f32_plan(batch, lq, lk, heads, head_dim).parts);
+}
 
 extern "C" size_t idolq_attention_workspace(int dtype, int64_t batch, int64_t lk, int64_t heads, int64_t head_dim) {
     return attn_workspace_bytes(dtype, batch, lk, heads, head_dim);
@@ -770,10 +763,11 @@ extern "C" int idolq_attention_ws(const void* q, const void* k, const void* v, i
     if (!q || !k || !v || !out) return fail(IDOLQ_EINVAL, "q, k, v and out must be non-null");
     AttnParams p{q, k, v, out, dtype, out_dtype, lq, lk, heads, head_dim, ldq, ldkv, q_bs, kv_bs, ldo, o_bs,
                  1.4426950408889634f / sqrtf((float)head_dim)};
-    p.out_vec = out_dtype == dtype && dtype != IDOLQ_F32 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
-                (ldo * 2) % 16 == 0 && (o_bs * 2) % 16 == 0;
+    p.batch = batch;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const size_t esz = dtype_size(dtype);
+    p.out_vec = out_dtype == dtype && reinterpret_cast<uintptr_t>(out) % 16 == 0 && (ldo * esz) % 16 == 0 &&
+                (o_bs * esz) % 16 == 0;
     const bool aligned = reinterpret_cast<uintptr_t>(q) % 16 == 0 && reinterpret_cast<uintptr_t>(k) % 16 == 0 &&
                          reinterpret_cast<uintptr_t>(v) % 16 == 0 && (ldq * esz) % 16 == 0 &&
                          (ldkv * esz) % 16 == 0 && (q_bs * esz) % 16 == 0 && (kv_bs * esz) % 16 == 0;
@@ -802,7 +796,12 @@ extern "C" int idolq_attention_ws(const void* q, const void* k, const void* v, i
             hipLaunchKernelGGL(attn_mfma_hd64<_Float16>, grid, dim3(256), 0, s, p);
         return check_launch("attn_mfma_hd64");
     }
-    if (dtype == IDOLQ_F32 && (head_dim == 32 || head_dim == 64) && aligned) {
+    if (f32_matrix(dtype, head_dim) && aligned) {
+        const AttnF32Plan plan = attn_f32_plan(batch, lq, lk, heads, head_dim);
+        const size_t need = attn_f32_workspace_bytes(batch, lq, heads, head_dim, plan.parts);
+        const bool given = need && workspace && workspace_bytes >= need && reinterpret_cast<uintptr_t>(workspace) % 16 == 0;
+        if (plan.waves && (plan.parts == 1 || given) && ldkv < ((int64_t)1 << 23))
+            return launch_attn_f32_split(p, plan, static_cast<float*>(workspace), s);
         const dim3 grid((unsigned)((lq + 31) / 32), (unsigned)heads, (unsigned)batch);
         if (head_dim == 64)
             hipLaunchKernelGGL(attn_f32_mfma<64>, grid, dim3(256), 0, s, p);

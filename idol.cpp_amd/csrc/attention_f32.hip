@@ -1,0 +1,594 @@
+// fp32 attention on the fp16 matrix cores: every fp32 operand as the sum of two fp16 values.
+//
+// The fp32 matrix instructions (v_mfma_f32_32x32x2_f32) take 64 cycles for the products the fp16 ones do in 4, so an
+// fp32 product made of three fp16 products has 5 times the rate. x = h + l with h = fp16(x) and l = fp16(x - h), both
+// rounded to nearest (x - h is exact in fp32), holds 22 to 24 bits of x; a product keeps hh, hl and lh and drops ll,
+// at most 2^-22 of it. Everything is accumulated in fp32, a rounding per 16 products where the fp32 instruction
+// rounds after 2, so the result is closer to fp64 than that kernel's over the sizes that were measured (64 to 8192
+// keys). Powers of two keep the operands
+// in fp16's range: one per query of Q, per key place of K, per column of V, and 2^4 for the probabilities (more would
+// cost the exponent's argument bits). So a value of Q, K or V loses bits of its low part only below 2^-12 of the
+// largest of its row or column, a probability below 2^-7 of its query's largest, and what is lost is below 2^-34 and
+// 2^-29 of that largest.
+//
+// attn_f32_split<HD, NW>: a workgroup of NW waves owns 32 NW queries of one (batch, head) and a range of 32-key tiles. The tile's K and V are split once per workgroup on their way into LDS (K planes [key][d],
+// V planes transposed [d][key], the keys of a 16-chunk in the order in which a lane of the score accumulator holds
+// them), two tile buffers, one barrier per tile. Scores are computed transposed, S^T = K Q^T, so a lane holds 16
+// scores of one query and its probabilities, split in registers, are the B operand of O^T = V^T P^T.
+//
+// Scales: a tile is staged with the scales of the one before it, and each wave votes whether they still fit (largest
+// magnitude of its values between 2^9 and 65000 after scaling). Where they do not, the workgroup takes new ones and
+// stages the tile again after the barrier (rare path, uniform over the workgroup); o moves to V's new scales exactly.
+// Infinite inputs, and K or Q of 2^60 and more, have no split: a workgroup that meets one starts its part again with
+// the fp32 matrix instructions on the inputs themselves (plain_part), so that infinities go through the arithmetic of
+// the plain fp32 product. A NaN splits into two and needs no path of its own.
+//
+// 1000 queries x 8192 keys x 16 heads of 64: 124 us (270 TFLOP/s), attn_f32_mfma 367 (92); 2-norm error against fp64
+// 5.6e-7, there 8.7e-7. The MFMAs of a tile and wave take 768 cycles and its vector instructions about 800 (counters:
+// hardly any of the two overlap), so what is left is mostly their sum: with 4 waves, whose staging is shared by half as
+// many queries, the same call takes 139 us, with a maximum per tile and one scale per tile 15% more.
+//
+// The key range is cut into parts (attn_f32_plan) where the query tiles alone leave CUs idle: each part writes its
+// maxima, sums and unnormalized output, and attn_f32_combine merges them.
+#include "attention.h"
+
+#include "q8_dma.h"
+
+namespace idolq {
+namespace {
+
+constexpr int kTile = 32;       // keys per tile
+constexpr int kVP = kTile + 8;  // elements per d row of a V plane (80 bytes: conflict-free 16-byte reads)
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+constexpr float kSplitLimit = 1152921504606846976.0f;  // 2^60
+constexpr float kScaledMin = 512.0f, kScaledMax = 65000.0f;
+// The probabilities are 2^(score + kOffset - maximum); a lane's 16 of a tile sum to less than 2^kSumBits, and to no more
+// than 2^(4 + kOffset) once the maximum is the largest.
+constexpr float kOffset = 4.0f;
+constexpr int kSumBits = 9;
+
+// Two values as fp16 pairs h, l.
+__device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& l) {
+    const f16x2 hv = __builtin_convertvector((f32x2{a, b}), f16x2);
+    const float ra = fmaf((float)hv.x, -1.0f, a), rb = fmaf((float)hv.y, -1.0f, b);
+    h = __builtin_bit_cast(uint32_t, hv);
+    l = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{ra, rb}), f16x2));
+}
+
+// 2^e as fp32, e within [-126, 127]
+__device__ __forceinline__ float pow2(int e) { return __builtin_bit_cast(float, (uint32_t)(127 + e) << 23); }
+
+// The exponent that takes a largest magnitude to [2^13, 2^14): 0 for 0, infinities and NaN, at most 74 (magnitudes
+// below 2^-61 keep fewer bits: their products are below 2^-100).
+__device__ __forceinline__ int scale_exp(float mx) {
+    const int e = 13 + 127 - (int)(__builtin_bit_cast(uint32_t, mx) >> 23);
+    return mx > 0.0f && mx < INFINITY ? (e < 74 ? e : 74) : 0;
+}
+
+__device__ __forceinline__ f32x16 mfma(f16x8 a, f16x8 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+// part_o [parts][batch][heads][lq][HD] unnormalized outputs, part_ml [...][lq][2] their maxima (base-2 domain) and sums
+template <int HD, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int qblocks, int parts, int per,
+                                                             float* __restrict__ part_o,
+                                                             float* __restrict__ part_ml) {
+    constexpr int kBQ = 32 * NW;  // queries per workgroup
+    constexpr int HH = HD / 2;    // depth per lane half of the fp32 instruction
+    constexpr int DC = HD / 16;   // 16-deep chunks of the scores
+    constexpr int DB = HD / 32;   // 32-wide d blocks of the output
+    constexpr int EV = kTile * HD / (64 * NW);  // staged values per thread of K and of V
+    constexpr int KP = HD + 8;    // elements per key row of a K plane (conflict-free 16-byte reads)
+    __shared__ __attribute__((aligned(16))) uint16_t k_lds[2][2][kTile * KP];
+    __shared__ __attribute__((aligned(16))) uint16_t v_lds[2][2][HD * kVP];
+    __shared__ uint32_t vote[2][NW];
+    __shared__ uint32_t col_max[2][HD];  // V's and o's largest finite magnitudes per column (their bits)
+    __shared__ int col_move[HD];         // the exponent by which o's column moves
+    __shared__ float col_unit[HD];       // what o's column is in units of
+    __shared__ float key_unit[kTile];    // the same of the scores of a key place
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int col = lane & 31, half = lane >> 5;
+    // Workgroups go to the 8 XCDs in turn; the query blocks of one (batch, head, part) read the same keys, so where
+    // the number of those groups allows it they are dealt to one XCD, whose L2 then serves the repeats.
+    const int64_t groups = p.batch * p.heads * parts;
+    int64_t g, qb;
+    if (groups % 8 == 0) {
+        const int64_t j = blockIdx.x >> 3;
+        qb = j % qblocks;
+        g = j / qblocks * 8 + (blockIdx.x & 7);
+    } else {
+        qb = blockIdx.x % qblocks;
+        g = blockIdx.x / qblocks;
+    }
+    const int64_t part = g % parts, bh = g / parts, h = bh % p.heads, b = bh / p.heads;
+    const int64_t lq = p.lq, lk = p.lk, ldkv = p.ldkv;
+    const int64_t q0 = qb * kBQ + wave * 32, qi = q0 + col;
+    const bool active = q0 < lq;  // wave-uniform: the others only stage
+    const float* qbase = static_cast<const float*>(p.q) + b * p.q_bs + h * HD;
+    const float* kbase = static_cast<const float*>(p.k) + b * p.kv_bs + h * HD;
+    const float* vbase = static_cast<const float*>(p.v) + b * p.kv_bs + h * HD;
+
+    // Q^T operand planes: the lane's query, d = 16 c + 8 half + e, times the query's 2^qe
+    f16x8 qf[2][DC];
+    float qmax = 0.0f;
+    {
+        const float* qrow = qbase + (qi < lq ? qi : lq - 1) * p.ldq;
+        float x[HH];
+#pragma unroll
+        for (int i = 0; i < HH; i += 4) {
+            const f32x4 a = *reinterpret_cast<const f32x4*>(qrow + 16 * (i >> 3) + 8 * half + (i & 4));
+            x[i] = a[0], x[i + 1] = a[1], x[i + 2] = a[2], x[i + 3] = a[3];
+            qmax = fmaxf(qmax, fmaxf(fmaxf(fabsf(a[0]), fabsf(a[1])), fmaxf(fabsf(a[2]), fabsf(a[3]))));
+        }
+        qmax = fmaxf(qmax, __shfl_xor(qmax, 32));
+        const float qs = pow2(scale_exp(qmax));
+#pragma unroll
+        for (int c = 0; c < DC; ++c) {
+            uint32_t w[2][4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) split2(x[8 * c + 2 * e] * qs, x[8 * c + 2 * e + 1] * qs, w[0][e], w[1][e]);
+#pragma unroll
+            for (int pl = 0; pl < 2; ++pl)
+                qf[pl][c] = __builtin_bit_cast(f16x8, make_uint4(w[pl][0], w[pl][1], w[pl][2], w[pl][3]));
+        }
+    }
+    // a score's factor to the base-2 domain is cq times its key's unit: ck for the 16 the lane holds
+    const float cq = p.scale_log2 * pow2(-scale_exp(qmax));
+
+    const int64_t tiles = (lk + kTile - 1) / kTile;
+    const int64_t t0 = part * per, t1 = t0 + per < tiles ? t0 + per : tiles;
+    float mc = -INFINITY, l_part = 0.0f;  // the running maximum (base-2 domain) and this lane's half of the sum
+    int ke = 0, ve = 0;  // the exponents of the scales of the thread's key of K and column of V
+    float ck[16];
+    f32x16 o[DB];
+#pragma unroll
+    for (int t = 0; t < DB; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[t][r] = 0.0f;
+
+    // Staging. K: thread t takes EV values of a key, a row to HD / EV consecutive threads. V: thread t takes d row t % HD
+    // and EV keys whose places in that row of the plane are contiguous: place 16 kc + 8 half + e holds key 16 kc +
+    // 8 (e / 4) + 4 half + e % 4.
+    const int skey = tid / (HD / EV), sd = EV * (tid % (HD / EV));
+    const int vd = tid % HD, vplace = tid / HD * EV;
+    const int vkey = (vplace >> 4) * 16 + ((vplace >> 2) & 1) * 8 + ((vplace >> 3) & 1) * 4 + (vplace & 3);
+    // a full tile's loads: per-thread byte offsets that no tile changes from a base that only the tile moves (both the
+    // base and a V key's row offset are scalar); the host keeps 32 rows below 2^31 bytes
+    const int koff = (int)(skey * ldkv + sd) * 4, voff = (int)(vkey * ldkv + vd) * 4;
+    float kr[EV], vr[EV];
+    auto load_tile = [&](int64_t t) __attribute__((always_inline)) {
+        const int64_t k0 = t * kTile;
+        if (k0 + kTile <= lk) {
+            const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<float*>(kbase + k0 * ldkv), 0, 0x7fffffff, 0x00020000);
+            const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<float*>(vbase + k0 * ldkv), 0, 0x7fffffff, 0x00020000);
+            if constexpr (EV == 2) {
+                const uint64_t v = __builtin_bit_cast(uint64_t, __builtin_amdgcn_raw_buffer_load_b64(rk, koff, 0, 0));
+                kr[0] = __builtin_bit_cast(float, (uint32_t)v), kr[1] = __builtin_bit_cast(float, (uint32_t)(v >> 32));
+            } else {
+#pragma unroll
+                for (int i = 0; i < EV; i += 4) {
+                    const f32x4 v =
+                        __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, koff + 4 * i, 0, 0));
+                    kr[i] = v[0], kr[i + 1] = v[1], kr[i + 2] = v[2], kr[i + 3] = v[3];
+                }
+            }
+            const int row = (int)ldkv * 4;
+#pragma unroll
+            for (int i = 0; i < EV; ++i)
+                vr[i] = __builtin_bit_cast(
+                    float, __builtin_amdgcn_raw_buffer_load_b32(rv, voff, ((i >> 2) * 8 + (i & 3)) * row, 0));
+        } else {  // the last tile: keys past lk are 0 (their scores are masked)
+            const int64_t kk = k0 + skey;
+#pragma unroll
+            for (int i = 0; i < EV; ++i) kr[i] = kk < lk ? kbase[kk * ldkv + sd + i] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < EV; ++i) {
+                const int64_t vk = k0 + vkey + (i >> 2) * 8 + (i & 3);
+                vr[i] = vk < lk ? vbase[vk * ldkv + vd] : 0.0f;
+            }
+        }
+    };
+    // votes: 1 K beyond its scale's range, 2 some K within it, 4 some K not 0; 8, 16, 32 the same of V;
+    // 64 a value without a split (K of 2^60 or more, an infinite V; big: one of the wave's queries)
+    auto stage_tile = [&](int buf, bool big) __attribute__((always_inline)) {
+        const float ks = pow2(ke), vs = pow2(ve);
+        float kmax = 0.0f, vmax = 0.0f;
+        uint32_t w[2][EV / 2];
+        auto store = [&](uint16_t* dst, int pl) __attribute__((always_inline)) {
+            if constexpr (EV == 8)
+                *reinterpret_cast<uint4*>(dst) = make_uint4(w[pl][0], w[pl][1], w[pl][2], w[pl][3]);
+            else if constexpr (EV == 4)
+                *reinterpret_cast<uint2*>(dst) = make_uint2(w[pl][0], w[pl][1]);
+            else
+                *reinterpret_cast<uint32_t*>(dst) = w[pl][0];
+        };
+#pragma unroll
+        for (int e = 0; e < EV / 2; ++e) {
+            const float x = kr[2 * e] * ks, y = kr[2 * e + 1] * ks;
+            split2(x, y, w[0][e], w[1][e]);
+            kmax = fmaxf(kmax, fmaxf(fabsf(x), fabsf(y)));
+        }
+        store(&k_lds[buf][0][skey * KP + sd], 0);
+        store(&k_lds[buf][1][skey * KP + sd], 1);
+#pragma unroll
+        for (int e = 0; e < EV / 2; ++e) {
+            const float x = vr[2 * e] * vs, y = vr[2 * e + 1] * vs;
+            split2(x, y, w[0][e], w[1][e]);
+            vmax = fmaxf(vmax, fmaxf(fabsf(x), fabsf(y)));
+        }
+        store(&v_lds[buf][0][vd * kVP + vplace], 0);
+        store(&v_lds[buf][1][vd * kVP + vplace], 1);
+        auto any = [&](bool c) __attribute__((always_inline)) { return __builtin_amdgcn_ballot_w64(c) != 0; };
+        uint32_t bits = any(kmax >= kScaledMin) ? 2u : 0u;  // every lane takes part
+        bits |= any(kmax > kScaledMax) ? 1u : 0u;
+        bits |= any(kmax > 0.0f) ? 4u : 0u;
+        bits |= any(vmax > kScaledMax) ? 8u : 0u;
+        bits |= any(vmax >= kScaledMin) ? 16u : 0u;
+        bits |= any(vmax > 0.0f) ? 32u : 0u;
+        bits |= any(big || kmax * pow2(-ke) >= kSplitLimit || vmax == INFINITY) ? 64u : 0u;
+        if (lane == 0) vote[buf][wave] = bits;
+    };
+    // New scales from the largest finite magnitudes of the tile in kr and vr, o moved to them, and the tile staged into
+    // buffer buf with them. Every wave takes part; col_max is 0 before and after.
+    auto rescale_tile = [&](int buf, bool big) __attribute__((always_inline)) {
+        auto finite = [](float x) __attribute__((always_inline)) { return fabsf(x) < INFINITY ? fabsf(x) : 0.0f; };
+        auto bits = [](float x) __attribute__((always_inline)) { return __builtin_bit_cast(uint32_t, x); };
+        float km = 0.0f, vm = 0.0f;
+#pragma unroll
+        for (int i = 0; i < EV; ++i) {
+            km = fmaxf(km, finite(kr[i]));
+            vm = fmaxf(vm, finite(vr[i]));
+        }
+#pragma unroll
+        for (int off = 1; off < HD / EV; off <<= 1) km = fmaxf(km, __shfl_xor(km, off));
+        ke = scale_exp(km);
+        if (sd == 0) key_unit[skey] = pow2(-ke);
+        atomicMax(&col_max[0][vd], bits(vm));
+#pragma unroll
+        for (int t = 0; t < DB; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                atomicMax(&col_max[1][t * 32 + 8 * (r >> 2) + 4 * half + (r & 3)], bits(finite(o[t][r])));
+        __syncthreads();
+        // o stays below 2^101: against an o that large in its units, values the tile would need a finer scale for do
+        // not count
+        const int room = 100 + 127 - (int)(col_max[1][vd] >> 23);
+        int move = scale_exp(__builtin_bit_cast(float, col_max[0][vd])) - ve;
+        if (move > room) move = room;
+        ve += move;
+        if (tid < HD) col_move[vd] = move, col_unit[vd] = pow2(-ve);
+        __syncthreads();
+        if (tid < HD) col_max[0][vd] = 0, col_max[1][vd] = 0;
+#pragma unroll
+        for (int t = 0; t < DB; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = col_move[t * 32 + 8 * (r >> 2) + 4 * half + (r & 3)];  // up to 187: in two steps
+                o[t][r] = o[t][r] * pow2(m / 2) * pow2(m - m / 2);
+            }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ck[r] = cq * key_unit[8 * (r >> 2) + 4 * half + (r & 3)];
+        stage_tile(buf, big);
+        __syncthreads();  // the planes and votes are in place, col_max is clear
+    };
+
+    // MASK: the last tile, with fewer than 32 keys; FIRST: the part's first tile, whose largest score sets the maximum
+    auto compute = [&](int buf, int64_t k0, auto mask_tag, auto first_tag) __attribute__((always_inline)) {
+        constexpr bool MASK = decltype(mask_tag)::value, FIRST = decltype(first_tag)::value;
+        f32x16 s;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+        f16x8 kf[2][DC];
+#pragma unroll
+        for (int pl = 0; pl < 2; ++pl)
+#pragma unroll
+            for (int c4 = 0; c4 < DC; ++c4)
+                kf[pl][c4] = *reinterpret_cast<const f16x8*>(&k_lds[buf][pl][col * KP + 16 * c4 + 8 * half]);
+#pragma unroll
+        for (int c4 = 0; c4 < DC; ++c4) s = mfma(kf[0][c4], qf[1][c4], s);
+#pragma unroll
+        for (int c4 = 0; c4 < DC; ++c4) s = mfma(kf[1][c4], qf[0][c4], s);
+#pragma unroll
+        for (int c4 = 0; c4 < DC; ++c4) s = mfma(kf[0][c4], qf[0][c4], s);
+        if (MASK) {
+            const int valid = (int)(lk - k0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (8 * (r >> 2) + 4 * half + (r & 3) >= valid) s[r] = -INFINITY;
+        }
+        // The maximum mc (kept less kOffset) is the first tile's, raised only where a lane's probabilities of a tile
+        // sum to 2^kSumBits or more, infinity and NaN included: no maximum is taken of the other tiles, the sum is
+        // needed anyway, and every probability stays inside fp16 (a wave-uniform branch). While every score was -inf,
+        // mc is -inf and 0 is subtracted: no weight.
+        if (FIRST) {
+            float mx = -INFINITY;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r] * ck[r]);
+            mc = fmaxf(mx, __shfl_xor(mx, 32)) - kOffset;
+        }
+        const float sub = mc == -INFINITY ? 0.0f : mc;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = fmaf(s[r], ck[r], -sub);
+        f32x16 pr;
+        float lt;
+        auto probabilities = [&]() __attribute__((always_inline)) {
+            float l2[2] = {0.0f, 0.0f};
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                pr[r] = __builtin_amdgcn_exp2f(s[r]);
+                l2[r & 1] += pr[r];
+            }
+            lt = l2[0] + l2[1];
+        };
+        probabilities();
+        if (!FIRST && __builtin_amdgcn_ballot_w64(!(lt < (float)(1 << kSumBits)) || mc == -INFINITY) != 0) {
+            float mx = -INFINITY;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            const bool none = mc == -INFINITY;
+            const float delta = none || mx > kOffset ? mx - kOffset : 0.0f;
+            if (delta > -INFINITY) {  // else still no score above -inf
+                const float alpha = none ? 0.0f : __builtin_amdgcn_exp2f(-delta);
+                mc = sub + delta;
+                l_part *= alpha;
+#pragma unroll
+                for (int t = 0; t < DB; ++t)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[r] -= delta;
+            }
+            probabilities();
+        }
+        l_part += lt;
+#pragma unroll
+        for (int kc = 0; kc < 2; ++kc) {
+            uint32_t w[2][4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) split2(pr[8 * kc + 2 * e], pr[8 * kc + 2 * e + 1], w[0][e], w[1][e]);
+            f16x8 pf[2], vf[DB][2];
+#pragma unroll
+            for (int pl = 0; pl < 2; ++pl)
+                pf[pl] = __builtin_bit_cast(f16x8, make_uint4(w[pl][0], w[pl][1], w[pl][2], w[pl][3]));
+#pragma unroll
+            for (int t = 0; t < DB; ++t)
+#pragma unroll
+                for (int pl = 0; pl < 2; ++pl)
+                    vf[t][pl] = *reinterpret_cast<const f16x8*>(
+                        &v_lds[buf][pl][(t * 32 + col) * kVP + 16 * kc + 8 * half]);
+#pragma unroll
+            for (int t = 0; t < DB; ++t) o[t] = mfma(vf[t][0], pf[1], o[t]);
+#pragma unroll
+            for (int t = 0; t < DB; ++t) o[t] = mfma(vf[t][1], pf[0], o[t]);
+#pragma unroll
+            for (int t = 0; t < DB; ++t) o[t] = mfma(vf[t][0], pf[0], o[t]);
+        }
+    };
+
+    // The part with fp32 matrix instructions on operands read from memory; the wave on its own, no LDS.
+    auto plain_part = [&]() __attribute__((always_inline)) {
+        const float* qrow = qbase + (qi < lq ? qi : lq - 1) * p.ldq;
+        mc = -INFINITY, l_part = 0.0f;
+#pragma unroll
+        for (int t = 0; t < DB; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[t][r] = 0.0f;
+#pragma unroll 1
+        for (int64_t t = t0; t < t1; ++t) {
+            const int64_t k0 = t * kTile;
+            const float* krow = kbase + (k0 + col < lk ? k0 + col : lk - 1) * ldkv;
+            f32x16 s;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+#pragma unroll 1
+            for (int i = half * HH; i < half * HH + HH; ++i)
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(krow[i], qrow[i], s, 0, 0, 0);
+            float mx = -INFINITY;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                s[r] = k0 + 8 * (r >> 2) + 4 * half + (r & 3) < lk ? s[r] * p.scale_log2 : -INFINITY;
+                mx = fmaxf(mx, s[r]);
+            }
+            const float m_new = fmaxf(mc, fmaxf(mx, __shfl_xor(mx, 32)));
+            const float sub = m_new == -INFINITY ? 0.0f : m_new;  // every score so far -inf: no weight
+            const float alpha = __builtin_amdgcn_exp2f(mc - sub);
+            mc = m_new;
+            l_part *= alpha;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                s[r] = __builtin_amdgcn_exp2f(s[r] - sub);
+                l_part += s[r];
+            }
+#pragma unroll
+            for (int d = 0; d < DB; ++d)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int64_t key = k0 + 8 * (r >> 2) + 4 * half + (r & 3);
+#pragma unroll
+                for (int d = 0; d < DB; ++d)
+                    o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(key < lk ? vbase[key * ldkv + d * 32 + col] : 0.0f, s[r],
+                                                                o[d], 0, 0, 0);
+            }
+        }
+    };
+
+    if (tid < HD) col_max[0][tid] = 0, col_max[1][tid] = 0, col_unit[tid] = 1.0f;
+    if (t0 < t1) load_tile(t0);
+    __syncthreads();
+    if (t0 < t1) rescale_tile(0, qmax >= kSplitLimit);
+    int buf = 0;
+    bool plain = false;  // uniform over the workgroup
+    // tile t (in buffer buf): its scales checked, the next tile's loads, the product, the next tile's staging and the
+    // barrier that publishes it; false where the part has to start again
+    auto step = [&](int64_t t, auto mask_tag, auto first_tag) __attribute__((always_inline)) {
+        uint32_t votes = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) votes |= vote[buf][w];
+        votes = __builtin_amdgcn_readfirstlane(votes);
+        if (votes & 64u) return false;
+        if ((votes & 9u) || (votes & 6u) == 4u || (votes & 48u) == 32u) rescale_tile(buf, false);
+        if (t + 1 < t1) load_tile(t + 1);
+        if (active) compute(buf, t * kTile, mask_tag, first_tag);
+        if (t + 1 < t1) stage_tile(buf ^ 1, false);
+        __syncthreads();
+        buf ^= 1;
+        return true;
+    };
+    const int64_t full = t1 * kTile <= lk ? t1 : t1 - 1;  // the last tile of all may hold fewer keys
+    if (t0 < t1) {
+        if (full > t0)
+            plain = !step(t0, std::false_type{}, std::true_type{});
+        else
+            plain = !step(t0, std::true_type{}, std::true_type{});
+        for (int64_t t = t0 + 1; t < full && !plain; ++t) plain = !step(t, std::false_type{}, std::false_type{});
+        if (full < t1 && full > t0 && !plain) plain = !step(full, std::true_type{}, std::false_type{});
+    }
+    // the factor that takes a sum of weights to weights of at most 1, and the maximum those refer to
+    float w = pow2(-kSumBits);
+    mc += (float)kSumBits;
+    if (plain) {
+        w = 1.0f;
+        if (active) plain_part();
+    }
+    auto unit = [&](int d) __attribute__((always_inline)) { return plain ? 1.0f : col_unit[d]; };
+
+    const float l = l_part + __shfl_xor(l_part, 32);
+    if (qi >= lq) return;
+    if (parts > 1) {
+        const int64_t row = ((part * p.batch + b) * p.heads + h) * lq + qi;
+#pragma unroll
+        for (int t = 0; t < DB; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4) {
+                const int d = t * 32 + 2 * r + 4 * half;
+                f32x4 v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = o[t][r + e] * w * unit(d + e);
+                *reinterpret_cast<f32x4*>(part_o + row * HD + d) = v;
+            }
+        if (half == 0) *reinterpret_cast<f32x2*>(part_ml + 2 * row) = f32x2{mc, l * w};
+        return;
+    }
+    const float inv = 1.0f / l;
+    const int64_t obase = b * p.o_bs + qi * p.ldo + h * HD;
+#pragma unroll
+    for (int t = 0; t < DB; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) {
+            const int d = t * 32 + 2 * r + 4 * half;
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = o[t][r + e] * inv * unit(d + e);
+            if (p.out_vec) {
+                *reinterpret_cast<f32x4*>(static_cast<float*>(p.out) + obase + d) = f32x4{v[0], v[1], v[2], v[3]};
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) store_from_float(p.out, p.out_dt, obase + d + e, v[e]);
+            }
+        }
+}
+
+// out = sum_s O_s 2^(m_s - m*) / sum_s l_s 2^(m_s - m*) over the parts; a wave per (batch, head, query) row: HD / 4
+// lanes of 4 columns each, the parts dealt to the 64 / (HD / 4) groups of lanes, whose sums meet through shuffles (a
+// fixed order). Reads every partial once; with the parts in groups their loads are in flight together.
+template <int HD>
+__global__ __launch_bounds__(256) void attn_f32_combine(AttnParams p, int parts, const float* __restrict__ part_o,
+                                                        const float* __restrict__ part_ml) {
+    constexpr int TPR = HD / 4, G = 64 / TPR;
+    const int64_t rows = p.batch * p.heads * p.lq;
+    const int64_t row = blockIdx.x * (int64_t)4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const int lane = threadIdx.x & 63, group = lane / TPR, d = 4 * (lane % TPR);
+    float mstar = -INFINITY, lsum = 0.0f;
+    for (int s = lane; s < parts; s += 64) mstar = fmaxf(mstar, part_ml[2 * (s * rows + row)]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) mstar = fmaxf(mstar, __shfl_xor(mstar, off));
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+    for (int s = group; s < parts; s += G) {
+        const f32x2 ml = *reinterpret_cast<const f32x2*>(part_ml + 2 * (s * rows + row));
+        const f32x4 v = *reinterpret_cast<const f32x4*>(part_o + (s * rows + row) * HD + d);
+        // a part whose scores are all -inf has no weight (its sums are 0 unless NaN, which is kept)
+        const float wgt = ml.x == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(ml.x - mstar);
+        lsum = fmaf(ml.y, wgt, lsum);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = fmaf(v[e], wgt, acc[e]);
+    }
+#pragma unroll
+    for (int off = TPR; off < 64; off <<= 1) {
+        lsum += __shfl_xor(lsum, off);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] += __shfl_xor(acc[e], off);
+    }
+    if (group != 0) return;
+    const float inv = 1.0f / lsum;
+    const int64_t q = row % p.lq, bh = row / p.lq;
+    const int64_t at = bh / p.heads * p.o_bs + q * p.ldo + bh % p.heads * HD + d;
+    if (p.out_vec) {
+        *reinterpret_cast<f32x4*>(static_cast<float*>(p.out) + at) = acc * inv;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) store_from_float(p.out, p.out_dt, at + e, acc[e] * inv);
+    }
+}
+
+}  // namespace
+
+// The cheapest of the kernel's forms (waves per workgroup), numbers of parts and, with waves 0, attn_f32_mfma, from
+// measured times in microseconds at head_dim 64: a tile step of a workgroup alone on its CU, of two (4 waves) and of
+// the 8-wave form, one and a half steps to start, and the merge (a launch and the partials written and read back);
+// attn_f32_mfma steps 32 keys in each of its 4 waves in 2.85, without the split's start. 300 queries, 16 heads, 64 /
+// 231 / 700 keys (this kernel against that one): 9.8 / 16.4 / 17.6 against 8.2 / 12.7 / 30 us.
+AttnF32Plan attn_f32_plan(int64_t batch, int64_t lq, int64_t lk, int64_t heads, int64_t head_dim) {
+    const int64_t cus = cu_count(), tiles = (lk + kTile - 1) / kTile;
+    const double depth = head_dim == 64 ? 1.0 : 0.75;
+    AttnF32Plan best{0, 1};
+    double best_cost = 0.5 + 2.85 * head_dim / 64 * ((tiles + 3) / 4) *
+                                 (((lq + 31) / 32 * heads * batch + cus - 1) / cus);
+    for (int nw = 4; nw <= 8; nw += 4) {
+        const int64_t base = (lq + 32 * nw - 1) / (32 * nw) * heads * batch, slots = nw == 4 ? 2 * cus : cus;
+        for (int s = 1; s <= 64 && s <= tiles && (s == 1 || s * base <= slots); ++s) {
+            const int64_t per = (tiles + s - 1) / s, wgs = s * base;
+            if (s > 1 && (tiles + per - 1) / per != s) continue;  // every part has tiles
+            const double step = depth * (nw == 8 ? 1.9 : wgs <= cus ? 1.5 : 2.2);
+            const double merge = s == 1 ? 0.0 : 4.0 + 0.005 * nw * wgs;
+            const double cost = (per + 1.5) * step * ((wgs + slots - 1) / slots) + merge;
+            if (cost < best_cost) best = {nw, s}, best_cost = cost;
+        }
+    }
+    return best;
+}
+
+size_t attn_f32_workspace_bytes(int64_t batch, int64_t lq, int64_t heads, int64_t head_dim, int parts) {
+    return parts <= 1 ? 0 : (size_t)parts * batch * heads * lq * (head_dim + 2) * sizeof(float);
+}
+
+int launch_attn_f32_split(const AttnParams& p, AttnF32Plan plan, float* workspace, hipStream_t s) {
+    const int64_t bq = 32 * plan.waves, qblocks = (p.lq + bq - 1) / bq, rows = p.batch * p.heads * p.lq;
+    const int64_t tiles = (p.lk + kTile - 1) / kTile, grid = qblocks * p.batch * p.heads * plan.parts;
+    const int64_t per = (tiles + plan.parts - 1) / plan.parts;
+    if (grid > 0x7fffffff || per > 0x7fffffff) return fail(IDOLQ_EINVAL, "grid too large");
+    float* part_ml = plan.parts > 1 ? workspace + (size_t)plan.parts * rows * p.head_dim : nullptr;
+    const dim3 g((unsigned)grid), block((unsigned)(64 * plan.waves));
+    const auto kernel = p.head_dim == 64 ? (plan.waves == 8 ? attn_f32_split<64, 8> : attn_f32_split<64, 4>)
+                                         : (plan.waves == 8 ? attn_f32_split<32, 8> : attn_f32_split<32, 4>);
+    hipLaunchKernelGGL(kernel, g, block, 0, s, p, (int)qblocks, plan.parts, (int)per, workspace, part_ml);
+    const int rc = check_launch("attn_f32_split");
+    if (rc || plan.parts <= 1) return rc;
+    const dim3 cgrid((unsigned)((rows + 3) / 4));
+    hipLaunchKernelGGL(p.head_dim == 64 ? attn_f32_combine<64> : attn_f32_combine<32>, cgrid, dim3(256), 0, s, p,
+                       plan.parts, workspace, part_ml);
+    return check_launch("attn_f32_combine");
+}
+
+}  // namespace idolq

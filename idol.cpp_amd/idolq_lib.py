@@ -47,6 +47,7 @@ _SIGNATURES = {
     "idolq_attention_ws": (_int, [_vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp,
                                   _int, _i64, _i64, _vp, _sz, _vp]),
     "idolq_attention_workspace": (_sz, [_int, _i64, _i64, _i64, _i64]),
+    "idolq_attention_f32_workspace": (_sz, [_i64, _i64, _i64, _i64, _i64]),
     "idolq_activation": (_int, [_vp, _int, _i64, _int, _vp]),
     "idolq_pos_embed": (_int, [_vp, _i64, _vp, _i64, _vp, _int, _i64, _vp]),
     "idolq_point_mlp": (_int, [_vp, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp,
@@ -392,10 +393,15 @@ def attention(q, k, v, batch, lq, lk, heads, head_dim, ldq, ldkv, q_bs, kv_bs, o
     dev = _require_cuda(q, k, v, out)
     if not (q.dtype == k.dtype == v.dtype):
         raise ValueError("q, k and v must share a dtype")
-    if staged_v is None:
-        staged_v = lk >= STAGED_V_MIN_KEYS
-    need = int(lib.idolq_attention_workspace(_code(q), batch, lk, heads, head_dim)) if staged_v else 0
-    ws = _attention_workspace(q.device, need) if need else None
+    if q.dtype == torch.float32:
+        # the parts of a cut key range: from the allocator's stream-ordered pool for this call alone
+        need = int(lib.idolq_attention_f32_workspace(batch, lq, lk, heads, head_dim))
+        ws = torch.empty(need, device=q.device, dtype=torch.uint8) if need else None
+    else:
+        if staged_v is None:
+            staged_v = lk >= STAGED_V_MIN_KEYS
+        need = int(lib.idolq_attention_workspace(_code(q), batch, lk, heads, head_dim)) if staged_v else 0
+        ws = _attention_workspace(q.device, need) if need else None
     _check(lib.idolq_attention_ws(_ptr(q), _ptr(k), _ptr(v), _code(q), batch, lq, lk, heads, head_dim, ldq, ldkv,
                                   q_bs, kv_bs, _ptr(out), _code(out), ldo, o_bs, _ptr(ws), need, _stream(dev)))
     return out

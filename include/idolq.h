@@ -185,6 +185,12 @@ int idolq_attention_ws(const void* q, const void* k, const void* v, int dtype, i
 /* Workspace bytes idolq_attention_ws uses for these shapes: the fp16 V^T tiles (batch x heads x ceil(lk / 64) tiles
  * of 8 KiB) and their exponents for bf16 inputs with head_dim 64; 0 for every other call. */
 size_t idolq_attention_workspace(int dtype, int64_t batch, int64_t lk, int64_t heads, int64_t head_dim);
+/* Workspace bytes (16-byte aligned, no zero-fill) with which idolq_attention_ws cuts the key range of an fp32 call
+ * with head_dim 32 or 64 into parts that fill the device (each part's maxima, sums and unnormalized output, merged by
+ * a second launch); 0 where the query tiles fill it alone and for every other head_dim. Without the workspace such a
+ * call runs a kernel that cuts the keys inside the workgroup.
+ * Same reference interface as idolq_attention (src/kernels.hpp:81-84). */
+size_t idolq_attention_f32_workspace(int64_t batch, int64_t lq, int64_t lk, int64_t heads, int64_t head_dim);
 
 /* In-place activation over count values: tanh-GELU (src/decoders.cpp:55-71 gelu_tanh), erf-GELU
  * (src/kernels.cpp:826-850) or ReLU. */

@@ -401,3 +401,116 @@ def test_attention_workspace_entry_point_through_the_c_abi():
         outs.append(out)
     torch.cuda.synchronize()
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+def _attention64(q, k, v, heads, hd):
+    out = np.empty(q.shape, np.float64)
+    for h in range(heads):
+        cols = slice(h * hd, (h + 1) * hd)
+        with np.errstate(all="ignore"):
+            s = q[:, cols].astype(np.float64) @ k[:, cols].astype(np.float64).T / np.sqrt(hd)
+            p = np.exp(s - s.max(axis=1, keepdims=True))
+            out[:, cols] = (p / p.sum(axis=1, keepdims=True)) @ v[:, cols].astype(np.float64)
+    return out
+
+
+@pytest.mark.parametrize("hd", [32, 64])
+@pytest.mark.parametrize("lq,lk,heads,batch", [(1, 1055, 8, 1), (127, 992, 2, 2), (128, 1025, 1, 1), (129, 1057, 3, 1),
+                                               (257, 2049, 4, 2), (40, 8192, 8, 1), (1000, 1500, 16, 1),
+                                               (1700, 90, 16, 1)])
+def test_attention_fp32_split_operands_match_fp64(hd, lq, lk, heads, batch):
+    # fp32 attention on bf16 triples, with and without a cut key range, groups a multiple of 8 or not: 24-bit operands
+    # and fp32 sums of 64 to 8192 terms against fp64: 2^-24 a rounding, at most lk / 16 + 64 of them in sequence, which
+    # grow like their square root: below 2e-6 at 8192 keys
+    rng = np.random.default_rng(lq * 7 + lk + hd)
+    dim = heads * hd
+    q = rng.normal(0, 1, (batch, lq, dim)).astype(np.float32)
+    kv = rng.normal(0, 1, (batch, lk, 2 * dim)).astype(np.float32)
+    kvd, out = to_dev(kv), torch.full((batch, lq, dim + 4), float("nan"), device=DEV)
+    L.attention(to_dev(q), kvd, kvd[:, :, dim:], batch, lq, lk, heads, hd, dim, 2 * dim, lq * dim, lk * 2 * dim, out,
+                dim + 4, lq * (dim + 4))
+    got = out.cpu().numpy()
+    assert np.all(np.isnan(got[:, :, dim:]))
+    for b in range(batch):
+        want = _attention64(q[b], kv[b, :, :dim], kv[b, :, dim:], heads, hd)
+        assert norm_rel(got[b, :, :dim], want) < 2e-6
+
+
+@pytest.mark.parametrize("hd", [32, 64])
+@pytest.mark.parametrize("lk", [40, 2000])
+def test_attention_fp32_split_operands_keep_infinities_and_large_values(hd, lk):
+    # keys masked by -inf in one channel (positive queries there), an infinite and a lowest-value V, scores beyond 2^60
+    # and a NaN: where the plain fp32 product is finite, infinite or NaN, so is this one
+    rng = np.random.default_rng(lk + hd)
+    lq, heads = 150, 8
+    dim = heads * hd
+    q = rng.normal(0, 1, (lq, dim)).astype(np.float32)
+    k = rng.normal(0, 1, (lk, dim)).astype(np.float32)
+    v = rng.normal(0, 1, (lk, dim)).astype(np.float32)
+    q[:, 0] = 1.0  # one bf16 value, so its low parts are 0
+    k[5, 0], k[lk - 1, 0] = -np.inf, -np.inf  # head 0: two keys without weight
+    v[7, hd + 3] = np.inf  # head 1: one infinite output column
+    v[9, 2 * hd] = np.finfo(np.float32).min  # head 2: the lowest value, finite times its weight
+    q[:, 3 * hd] = 2.0 ** 70  # head 3: one key takes every query
+    k[:, 3 * hd] = 0.0
+    k[11, 3 * hd] = 1.0
+    v[13, 4 * hd + 1] = np.nan  # head 4: one NaN column
+    k[:, 5 * hd] = -np.inf  # head 5: no key has weight
+    q[:, 5 * hd] = 1.0
+    q[3, 6 * hd] = np.inf  # head 6: one query without a result
+    out = torch.empty((lq, dim), device=DEV)
+    L.attention(to_dev(q), to_dev(k), to_dev(v), 1, lq, lk, heads, hd, dim, dim, 0, 0, out, dim, 0)
+    got = out.cpu().numpy().astype(np.float64)
+    keep = np.ones(lk, bool)
+    keep[[5, lk - 1]] = False
+    head = lambda h: slice(h * hd, (h + 1) * hd)
+    want = _attention64(q[:, head(0)], k[keep][:, head(0)], v[keep][:, head(0)], 1, hd)
+    assert norm_rel(got[:, head(0)], want) < 2e-6
+    assert np.all(got[:, hd + 3] == np.inf) and np.isfinite(got[:, hd:hd + 3]).all()
+    want = _attention64(q[:, head(2)], k[:, head(2)], v[:, head(2)], 1, hd)
+    assert norm_rel(got[:, 2 * hd] * 1e-30, want[:, 0] * 1e-30) < 1e-5 and norm_rel(got[:, 2 * hd + 1:3 * hd], want[:, 1:]) < 2e-6
+    assert np.array_equal(got[:, head(3)], np.broadcast_to(v[11, head(3)], (lq, hd)))
+    assert np.all(np.isnan(got[:, 4 * hd + 1])) and np.isfinite(got[:, 4 * hd + 2:5 * hd]).all()
+    assert np.all(np.isnan(got[:, head(5)]))
+    rest = np.arange(lq) != 3
+    assert np.all(np.isnan(got[3, head(6)])) and np.isfinite(got[rest][:, head(6)]).all()
+
+
+@pytest.mark.parametrize("hd", [32, 64])
+def test_attention_fp32_split_operands_hold_rows_and_columns_of_any_scale(hd):
+    # keys and columns of V whose magnitudes differ by powers of two up to 2^40 and change along the keys, so the
+    # operands' scales change again and again; zero keys and columns among them: each column of V against fp64 at the
+    # accuracy of equal scales
+    rng = np.random.default_rng(31 + hd)
+    lq, lk, heads = 200, 1500, 2
+    dim = heads * hd
+    q = rng.normal(0, 1, (lq, dim)).astype(np.float32) * np.exp2(rng.integers(-3, 1, (lq, 1))).astype(np.float32)
+    k = rng.normal(0, 1, (lk, dim)).astype(np.float32) * np.exp2(rng.integers(-30, 1, (lk, 1))).astype(np.float32)
+    v = rng.normal(0, 1, (lk, dim)).astype(np.float32) * np.exp2(rng.integers(-20, 21, (1, dim))).astype(np.float32)
+    v *= np.exp2(np.floor(np.arange(lk)[:, None] / 200.0)).astype(np.float32)
+    k[600:680] = 0.0
+    v[:, 5] = 0.0
+    out = torch.empty((lq, dim), device=DEV)
+    L.attention(to_dev(q), to_dev(k), to_dev(v), 1, lq, lk, heads, hd, dim, dim, 0, 0, out, dim, 0)
+    got, want = out.cpu().numpy(), _attention64(q, k, v, heads, hd)
+    assert not got[:, 5].any()
+    for d in range(dim):
+        if d != 5:
+            assert norm_rel(got[:, d], want[:, d]) < 2e-6, d
+
+
+def test_attention_fp32_without_a_workspace_takes_the_kernel_that_cuts_keys_inside():
+    # the C entry point without a workspace, where the split kernel would want one: the same result within fp32
+    lib = L.load()
+    rng = np.random.default_rng(5)
+    lq, lk, heads, hd = 70, 900, 4, 64
+    dim = heads * hd
+    q, k, v = (rng.normal(0, 1, (n, dim)).astype(np.float32) for n in (lq, lk, lk))
+    qd, kd, vd = to_dev(q), to_dev(k), to_dev(v)
+    assert lib.idolq_attention_f32_workspace(1, lq, lk, heads, hd) > 0
+    assert lib.idolq_attention_f32_workspace(1, lq, lk, heads, 48) == 0
+    out = torch.empty((lq, dim), device=DEV)
+    assert lib.idolq_attention(L._ptr(qd), L._ptr(kd), L._ptr(vd), L.F32, 1, lq, lk, heads, hd, dim, dim, 0, 0,
+                               L._ptr(out), L.F32, dim, 0, L._stream(DEV)) == 0
+    torch.cuda.synchronize()
+    assert norm_rel(out.cpu().numpy(), _attention64(q, k, v, heads, hd)) < 2e-6
