@@ -329,17 +329,19 @@ int quantize_act_launch(const void* x, int x_dtype, int64_t m, int64_t k, int64_
                         int32_t* qsum, hipStream_t stream) {
     const int64_t nb = k / kQ8Block;
     if (m * nb == 0) return IDOLQ_OK;
-    const bool vec16 = !qsum && (x_dtype == IDOLQ_BF16 || x_dtype == IDOLQ_F16) &&
-                       reinterpret_cast<uintptr_t>(x) % 16 == 0 && (ldx * 2) % 16 == 0 &&
+    const bool vec16 = !qsum && reinterpret_cast<uintptr_t>(x) % 16 == 0 && (ldx * dtype_size(x_dtype)) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(qa) % 8 == 0;
     if (vec16) {
         const dim3 grid((unsigned)((4 * m * nb + 255) / 256));
         if (x_dtype == IDOLQ_BF16)
             hipLaunchKernelGGL((quantize_act16_kernel<__bf16, false>), grid, dim3(256), 0, stream,
                                static_cast<const __bf16*>(x), m, nb, ldx, qa, scale, nullptr, 0);
-        else
+        else if (x_dtype == IDOLQ_F16)
             hipLaunchKernelGGL((quantize_act16_kernel<_Float16, false>), grid, dim3(256), 0, stream,
                                static_cast<const _Float16*>(x), m, nb, ldx, qa, scale, nullptr, 0);
+        else
+            hipLaunchKernelGGL((quantize_act16_kernel<float, false>), grid, dim3(256), 0, stream,
+                               static_cast<const float*>(x), m, nb, ldx, qa, scale, nullptr, 0);
         return check_launch("quantize_act16_kernel");
     }
     hipLaunchKernelGGL(quantize_act_kernel, dim3((unsigned)((m * nb + 255) / 256)), dim3(256), 0, stream, x, x_dtype, m,

@@ -9,12 +9,10 @@
 //      bytes de-interleaved into a code array (byte-aligned rows of 64 codes) and an fp32 scale array;
 //   3. MFMA over the two blocks. The next stage's global loads are in flight meanwhile.
 // Arithmetic (see idolq.h): DEQUANT converts codes to T(fp32(d) * q) and chains the MFMA accumulators over k;
-// EXACT feeds the codes exactly and folds each block's fp32 sum with its d; INT8 multiplies int8 activations by the
-// codes with v_mfma_i32_32x32x32_i8 and folds s_a * d per block.
+// EXACT feeds the codes exactly and folds each block's fp32 sum with its d. The INT8 mode is in q8_gemm_i8.hip.
 //
-// MFMA operand layout (32 x 32 tiles): lane l supplies row (or column) l % 32 and the 8 (bf16/fp16, 16-deep
-// instruction) or 16 (int8, 32-deep) consecutive k starting at (l / 32) * 8 (resp. 16); accumulator element r of
-// lane l is row 8 * (r / 4) + 4 * (l / 32) + r % 4, column l % 32.
+// MFMA operand layout (32 x 32 tiles): lane l supplies row (or column) l % 32 and the 8 consecutive k starting at
+// (l / 32) * 8; accumulator element r of lane l is row 8 * (r / 4) + 4 * (l / 32) + r % 4, column l % 32.
 #include "q8_gemm.h"
 
 #include <algorithm>
@@ -27,77 +25,6 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kKStep = 64;                // depth per stage: two Q8_0 blocks
 constexpr int kAPitch = kKStep + 8;       // 16-bit elements per activation row in LDS (144 bytes)
-constexpr int kCodePitch8 = kKStep + 16;  // bytes per row of int8 operands for 16-byte reads (80)
-
-// ------------------------------------------------------------------------------------------------ weight staging
-// Flat loader for the 68 bytes (two blocks) of each of BN weight rows per stage.
-template <int BN, bool W4>
-struct WeightStage {
-    static constexpr int kUnits = W4 ? BN * 17 : BN * 34;  // dwords or halfwords
-    static constexpr int kPer = (kUnits + kThreads - 1) / kThreads;
-    uint32_t v[kPer];
-
-    __device__ __forceinline__ void load(const GemmParams& p, int n0, int blk0, int nblocks) {
-        const int tid = threadIdx.x;
-#pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const int u = tid + i * kThreads;
-            v[i] = 0;
-            if (u < kUnits) {
-                const int row = W4 ? u / 17 : u / 34;
-                const int part = W4 ? u - row * 17 : u - row * 34;
-                const bool second = W4 ? part >= 9 : part >= 17;  // unit touches the second block only
-                if (n0 + row < p.n && (!second || blk0 + 1 < nblocks)) {
-                    const uint8_t* src = p.w + (int64_t)(n0 + row) * p.row_bytes + (int64_t)blk0 * kQ8Bytes;
-                    if (W4)
-                        v[i] = reinterpret_cast<const uint32_t*>(src)[part];
-                    else
-                        v[i] = reinterpret_cast<const uint16_t*>(src)[part];
-                }
-            }
-        }
-    }
-
-    // De-interleave into codes [BN][pitch] (int8) and scales [BN][2] (fp32).
-    template <int PITCH>
-    __device__ __forceinline__ void store(uint8_t* codes, float* scales) const {
-        const int tid = threadIdx.x;
-#pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const int u = tid + i * kThreads;
-            if (u >= kUnits) continue;
-            const uint32_t x = v[i];
-            if (W4) {
-                const int row = u / 17, part = u - row * 17;
-                uint8_t* c = codes + row * PITCH;
-                if (part == 0) {
-                    scales[row * 2] = half_bits_to_float((uint16_t)(x & 0xffff));
-                    *reinterpret_cast<uint16_t*>(c) = (uint16_t)(x >> 16);
-                } else if (part < 8) {
-                    *reinterpret_cast<uint16_t*>(c + 4 * part - 2) = (uint16_t)(x & 0xffff);
-                    *reinterpret_cast<uint16_t*>(c + 4 * part) = (uint16_t)(x >> 16);
-                } else if (part == 8) {
-                    *reinterpret_cast<uint16_t*>(c + 30) = (uint16_t)(x & 0xffff);
-                    scales[row * 2 + 1] = half_bits_to_float((uint16_t)(x >> 16));
-                } else {
-                    *reinterpret_cast<uint32_t*>(c + 4 * part - 4) = x;
-                }
-            } else {
-                const int row = u / 34, part = u - row * 34;
-                uint8_t* c = codes + row * PITCH;
-                const uint16_t h = (uint16_t)x;
-                if (part == 0)
-                    scales[row * 2] = half_bits_to_float(h);
-                else if (part < 17)
-                    *reinterpret_cast<uint16_t*>(c + 2 * part - 2) = h;
-                else if (part == 17)
-                    scales[row * 2 + 1] = half_bits_to_float(h);
-                else
-                    *reinterpret_cast<uint16_t*>(c + 2 * part - 4) = h;
-            }
-        }
-    }
-};
 
 // ------------------------------------------------------------------------------------------------ activation staging
 // BM rows x 64 k of x per stage in 16-byte units. The per-thread row offsets (in 16-byte units, ~0u for rows
@@ -334,34 +261,6 @@ __device__ __forceinline__ void convert_stage(const uint32_t* raw, uint16_t* b, 
 }
 
 // ------------------------------------------------------------------------------------------------ epilogue
-__device__ __forceinline__ void epilogue_store(const GemmParams& p, int row, int col, float v, float bias) {
-    if ((p.flags & IDOLQ_FLAG_ROUND_BEFORE_BIAS) != 0) v = round_through(p.y_dt, v);
-    v += bias;
-    if (p.res) v += load_as_float(p.res, p.res_dt, (int64_t)row * p.ldr + col);
-    v = apply_act(p.act, v);
-    store_from_float(p.y, p.y_dt, (int64_t)row * p.ldy + col, v);
-}
-
-template <int TM, int TN, int WM, int WN>
-__device__ __forceinline__ void write_tile(const GemmParams& p, const f32x16 (&acc)[TM][TN], int m0, int n0) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-#pragma unroll
-    for (int tn = 0; tn < TN; ++tn) {
-        const int col = n0 + wn * WN + tn * 32 + (lane & 31);
-        if (col >= p.n) continue;
-        const float bias = p.bias ? load_as_float(p.bias, p.bias_dt, col) : 0.0f;
-#pragma unroll
-        for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = m0 + wm * WM + tm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (row < p.m) epilogue_store(p, row, col, acc[tm][tn][r], bias);
-            }
-    }
-}
-
-
 // Epilogue through LDS: the accumulator tile is written to LDS as fp32 ([BM][BN + 4]), then each thread takes runs of
 // 8 consecutive columns of one row and applies the epilogue with vector loads of bias and residual and one 16-byte
 // (32-byte for fp32) store per run, so each wave writes whole row segments instead of 2-byte scattered stores.
@@ -616,121 +515,6 @@ __global__ __launch_bounds__(THREADS) void q8_gemm_kernel(GemmParams p) {
     write_tile_staged<BM, BN, TM, TN, WM, WN, THREADS, KS>(p, acc, m0, n0, reinterpret_cast<float*>(smem));
 }
 
-// ------------------------------------------------------------------------------------------------ int8 MFMA kernel
-// A = int8 activations (quantized per row and block by quantize_act_kernel) with fp32 scales per row and block.
-// DOTS stores the raw int32 block sums instead of folding them (the bit-exact test entry point).
-template <int BM, int BN, bool W4, bool DOTS>
-__global__ __launch_bounds__(kThreads) void q8_gemm_int8_kernel(GemmParams p) {
-    constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
-    constexpr int kAUnitsPerRow = kKStep / 16;  // 4 x 16 bytes of int8 per row per stage
-    constexpr int kAPer = BM * kAUnitsPerRow / kThreads;
-    static_assert(BM * kAUnitsPerRow % kThreads == 0, "tile size");
-
-    __shared__ __attribute__((aligned(16))) uint8_t a_lds[BM * kCodePitch8];
-    __shared__ __attribute__((aligned(16))) uint8_t code_lds[BN * kCodePitch8];
-    __shared__ float scale_lds[BN * 2];
-    __shared__ __attribute__((aligned(16))) float sa_lds[2][BM];
-
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    int tile_m, tile_n;
-    tile_coords(p.tiles_m, p.tiles_n, tile_m, tile_n);
-    const int m0 = tile_m * BM, n0 = tile_n * BN;
-    const int nblocks = p.k / kQ8Block;
-    const int nsteps = (nblocks + 1) / 2;
-
-    f32x16 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    WeightStage<BN, W4> ws;
-    uint4 av[kAPer];
-    float sav = 0.0f;
-    auto load_a = [&](int s) {
-        const int k0 = s * kKStep;
-#pragma unroll
-        for (int i = 0; i < kAPer; ++i) {
-            const int u = threadIdx.x + i * kThreads;
-            const int row = u / kAUnitsPerRow, cu = u - row * kAUnitsPerRow;
-            const int kk = k0 + cu * 16;
-            av[i] = make_uint4(0, 0, 0, 0);
-            if (m0 + row < p.m && kk < p.k) av[i] = *reinterpret_cast<const uint4*>(p.qa + (int64_t)(m0 + row) * p.k + kk);
-        }
-        sav = 0.0f;
-        if (!DOTS && threadIdx.x < 2 * BM) {
-            const int row = threadIdx.x >> 1, b = 2 * s + (threadIdx.x & 1);
-            if (m0 + row < p.m && b < nblocks) sav = p.sa[(int64_t)(m0 + row) * nblocks + b];
-        }
-    };
-    load_a(0);
-    ws.load(p, n0, 0, nblocks);
-
-    for (int s = 0; s < nsteps; ++s) {
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < kAPer; ++i) {
-            const int u = threadIdx.x + i * kThreads;
-            const int row = u / kAUnitsPerRow, cu = u - row * kAUnitsPerRow;
-            *reinterpret_cast<uint4*>(a_lds + row * kCodePitch8 + cu * 16) = av[i];
-        }
-        if (threadIdx.x < 2 * BM) sa_lds[threadIdx.x & 1][threadIdx.x >> 1] = sav;
-        ws.template store<kCodePitch8>(code_lds, scale_lds);
-        __syncthreads();
-        if (s + 1 < nsteps) {
-            load_a(s + 1);
-            ws.load(p, n0, 2 * (s + 1), nblocks);
-        }
-#pragma unroll
-        for (int blk = 0; blk < 2; ++blk) {
-            if (2 * s + blk >= nblocks) break;
-            i32x4 b[TN];
-            float dw[TN];
-#pragma unroll
-            for (int tn = 0; tn < TN; ++tn) {
-                const int col = wn * WN + tn * 32 + (lane & 31);
-                dw[tn] = scale_lds[col * 2 + blk];
-                b[tn] = *reinterpret_cast<const i32x4*>(code_lds + col * kCodePitch8 + blk * 32 + (lane >> 5) * 16);
-            }
-#pragma unroll
-            for (int tm = 0; tm < TM; ++tm) {
-                const int row = wm * WM + tm * 32 + (lane & 31);
-                const i32x4 a = *reinterpret_cast<const i32x4*>(a_lds + row * kCodePitch8 + blk * 32 + (lane >> 5) * 16);
-                f32x4 sa4[4];
-                if (!DOTS) {
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        sa4[q] = *reinterpret_cast<const f32x4*>(&sa_lds[blk][wm * WM + tm * 32 + 8 * q + 4 * (lane >> 5)]);
-                }
-#pragma unroll
-                for (int tn = 0; tn < TN; ++tn) {
-                    i32x16 zero;
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) zero[r] = 0;
-                    const i32x16 dots = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b[tn], zero, 0, 0, 0);
-                    if (DOTS) {
-                        const int col = n0 + wn * WN + tn * 32 + (lane & 31);
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            const int grow = m0 + wm * WM + tm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                            if (grow < p.m && col < p.n)
-                                p.dots[((int64_t)grow * p.n + col) * nblocks + 2 * s + blk] = dots[r];
-                        }
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < 16; ++r)
-                            acc[tm][tn][r] = fmaf((float)dots[r], sa4[r >> 2][r & 3] * dw[tn], acc[tm][tn][r]);
-                    }
-                }
-            }
-        }
-    }
-    if (!DOTS) write_tile<TM, TN, WM, WN>(p, acc, m0, n0);
-}
-
 // ------------------------------------------------------------------------------------------------ launch
 template <int BM, int BN, int THREADS>
 int launch_16bit_tile(GemmParams p, int xt, int mode, bool w4, hipStream_t stream) {
@@ -806,18 +590,6 @@ int launch_16bit(GemmParams p, int xt, int mode, bool w4, void* workspace, size_
     if (t.bm == 256) return launch_16bit_tile<256, 128, 512>(p, xt, mode, w4, stream);
     if (t.bn == 128) return launch_16bit_tile<128, 128, kThreads>(p, xt, mode, w4, stream);
     return launch_16bit_tile<128, 64, kThreads>(p, xt, mode, w4, stream);
-}
-
-template <int BM, int BN, bool DOTS>
-int launch_int8(GemmParams p, bool w4, hipStream_t stream) {
-    p.tiles_m = (p.m + BM - 1) / BM;
-    p.tiles_n = (p.n + BN - 1) / BN;
-    const dim3 grid(p.tiles_m * p.tiles_n), block(kThreads);
-    if (w4)
-        hipLaunchKernelGGL((q8_gemm_int8_kernel<BM, BN, true, DOTS>), grid, block, 0, stream, p);
-    else
-        hipLaunchKernelGGL((q8_gemm_int8_kernel<BM, BN, false, DOTS>), grid, block, 0, stream, p);
-    return check_launch("q8_gemm_int8_kernel");
 }
 
 }  // namespace
@@ -943,7 +715,7 @@ extern "C" int idolq_q8_0_gemm(const void* x, int x_dtype, int64_t m, int64_t k,
         if (rc) return rc;
         p.qa = qa;
         p.sa = sa;
-        return launch_int8<128, 128, false>(p, w4, s);
+        return launch_i8_rows(p, w4, s);
     }
     if (mode == IDOLQ_MODE_EXACT && tiled) {
         // x -> bf16 high and low parts (x - hi rounded to bf16) in the scratch, then two bf16 products per block
@@ -996,7 +768,7 @@ extern "C" int idolq_q8_0_block_dots(const int8_t* qa, int64_t m, int64_t k, con
     p.qa = qa;
     p.dots = dots;
     const bool w4 = p.row_bytes % 4 == 0 && (reinterpret_cast<uintptr_t>(p.w) & 3) == 0;
-    return launch_int8<128, 128, true>(p, w4, static_cast<hipStream_t>(stream));
+    return launch_i8_rows(p, w4, static_cast<hipStream_t>(stream));
 }
 
 // ------------------------------------------------------------------------------------------------ no-allocation GEMM

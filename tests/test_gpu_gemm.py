@@ -95,6 +95,28 @@ def test_int8_mfma_block_dots_are_bit_exact(m, n, k, off, cnt):
     assert np.array_equal(got, O.block_dots(qa, w, k, off, cnt))
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 33, 32), (16, 64, 160), (17, 63, 128), (65, 129, 224), (130, 64, 4096),
+                                   (2049, 2050, 96), (1, 4096, 256)])
+@pytest.mark.parametrize("skew", [0, 2])
+def test_int8_row_major_tiles_fold_block_by_block(m, n, k, skew):
+    # every tile of the row-major INT8 kernel (16 x 32, 64 x 64, 128 x 128), partial tiles, a last stage of 1 to 3
+    # blocks, weight rows 2 bytes off a dword, fp32 rows 4 bytes off 16 (the one-thread quantizer): the codes and
+    # scales of the oracle and its exact dots, folded in fp64: fp32 rounds once per block, below 1e-6 at 128 blocks
+    rng = np.random.default_rng(m + n + k)
+    a = rng.normal(0, 1, (m, k + 1)).astype(np.float32)
+    w = q8(rng, n, k, 0.05)
+    x = to_dev(a)[:, 1:] if skew else to_dev(np.ascontiguousarray(a[:, 1:]))
+    buf = torch.zeros(w.size + skew, dtype=torch.uint8, device=DEV)
+    buf[skew:] = to_dev(w.reshape(-1))
+    got = L.gemm(x, buf[skew:], n, mode=L.MODE_INT8, out_dtype=torch.float32).cpu().numpy()
+    qa, sa, _ = O.quantize_act(np.ascontiguousarray(a[:, 1:]))
+    blocks = w.reshape(n, k // 32, 34)
+    d = np.ascontiguousarray(blocks[:, :, :2]).view(np.float16)[:, :, 0].astype(np.float64)
+    xs = (qa.reshape(m, k // 32, 32) * np.asarray(sa, np.float64).reshape(m, k // 32, 1)).reshape(m, k)
+    ws = (blocks[:, :, 2:].view(np.int8) * d[:, :, None]).reshape(n, k)
+    assert norm_rel(got, xs @ ws.T) < 1e-6
+
+
 def test_gemm_against_reference_golden_vectors(golden):
     # The reference's own outputs for its test shapes (tests/golden/gemm_q8.npz): EXACT vs the float kernel and INT8
     # vs the integer kernel, fp32 in and out, each within 1e-5 norm-relative, on row-major Q8_0 blocks and (five of
