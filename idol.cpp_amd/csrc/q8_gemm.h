@@ -70,6 +70,9 @@ int launch_wide_i8(GemmParams p, void* workspace, size_t workspace_bytes, hipStr
 // The EXACT mode on tiled weights (p.x, p.x_lo: bf16 high and low parts of the activations, row stride k).
 int launch_wide_exact(GemmParams p, void* workspace, size_t workspace_bytes, hipStream_t stream);
 
+// The EXACT mode with fp32 activations on GGUF row-major weights (q8_gemm_exact.hip).
+int launch_exact_rows(const GemmParams& p, bool w4, hipStream_t stream);
+
 // The INT8 mode (and, with p.dots, its block sums) on GGUF row-major weights (q8_gemm_i8.hip): p.qa and p.sa row-major.
 int launch_i8_rows(const GemmParams& p, bool w4, hipStream_t stream);
 

@@ -5,15 +5,16 @@
 //   1. global -> registers: the activation tile with 16-byte loads, and the weight tile as a flat run of dwords
 //      (or halfwords when a row of blocks is not 4-byte aligned), consecutive lanes reading consecutive bytes of a
 //      row, so each row's 68 bytes are fetched as one coalesced span;
-//   2. registers -> LDS: activations as 16-bit MFMA operands (fp32 split into bf16 high + low parts), and the weight
+//   2. registers -> LDS: activations as 16-bit MFMA operands, and the weight
 //      bytes de-interleaved into a code array (byte-aligned rows of 64 codes) and an fp32 scale array;
 //   3. MFMA over the two blocks. The next stage's global loads are in flight meanwhile.
 // Arithmetic (see idolq.h): DEQUANT converts codes to T(fp32(d) * q) and chains the MFMA accumulators over k;
-// EXACT feeds the codes exactly and folds each block's fp32 sum with its d. The INT8 mode is in q8_gemm_i8.hip.
+// EXACT feeds the codes exactly and folds each block's fp32 sum with its d. The INT8 mode is in q8_gemm_i8.hip, EXACT
+// with fp32 activations in q8_gemm_exact.hip.
 //
 // MFMA operand layout (32 x 32 tiles): lane l supplies row (or column) l % 32 and the 8 consecutive k starting at
 // (l / 32) * 8; accumulator element r of lane l is row 8 * (r / 4) + 4 * (l / 32) + r % 4, column l % 32.
-#include "q8_gemm.h"
+#include "q8_epilogue.h"
 
 #include <algorithm>
 #include <mutex>
@@ -27,18 +28,14 @@ constexpr int kKStep = 64;                // depth per stage: two Q8_0 blocks
 constexpr int kAPitch = kKStep + 8;       // 16-bit elements per activation row in LDS (144 bytes)
 
 // ------------------------------------------------------------------------------------------------ activation staging
-// BM rows x 64 k of x per stage in 16-byte units. The per-thread row offsets (in 16-byte units, ~0u for rows
-// outside m) are computed once; a stage only adds its k offset. Unit u = tid + 256 i covers row u / kUnitsPerRow,
-// column unit tid % kUnitsPerRow (the same for every i).
-// XA: x is known to be 16-byte aligned (no runtime test, so the load sequence has no branch for the compiler's
-// wait counts to merge over).
-template <int BM, int XT, int THREADS, bool XA = false>
+// BM rows x 64 k of 16-bit x per stage in 16-byte units. The per-thread row offsets (in elements, ~0u for rows outside
+// m) are computed once; a stage only adds its k offset. Unit u = tid + THREADS i covers row u / 8, column unit tid % 8
+// (the same for every i).
+template <int BM, int THREADS>
 struct ActStage {
-    static constexpr int kEsz = XT == XT_F32 ? 4 : 2;
-    static constexpr int kUnitsPerRow = kKStep * kEsz / 16;  // 8 (16-bit) or 16 (fp32)
+    static constexpr int kUnitsPerRow = kKStep * 2 / 16, kElems = 8;
     static constexpr int kRowsPerPass = THREADS / kUnitsPerRow;
     static constexpr int kPer = BM / kRowsPerPass;
-    static constexpr int kElems = 16 / kEsz;
     static_assert(BM % kRowsPerPass == 0, "tile size");
     uint32_t off[kPer];  // element offset of the unit's row start + column unit, ~0u when the row is outside m
     uint4 v[kPer];
@@ -58,12 +55,12 @@ struct ActStage {
     __device__ __forceinline__ void load(const GemmParams& p, int k0) {
         const int kk = k0 + (threadIdx.x % kUnitsPerRow) * kElems;
         const bool kin = kk < p.k;
-        if (XA || p.x_aligned) {
+        const uint16_t* x = static_cast<const uint16_t*>(p.x);
+        if (p.x_aligned) {
 #pragma unroll
             for (int i = 0; i < kPer; ++i) {
                 ok[i] = off[i] != ~0u && kin;
-                const char* src = static_cast<const char*>(p.x) + (ok[i] ? ((size_t)off[i] + k0) * kEsz : 0);
-                v[i] = *reinterpret_cast<const uint4*>(src);
+                v[i] = *reinterpret_cast<const uint4*>(x + (ok[i] ? (size_t)off[i] + k0 : 0));
             }
             return;
         }
@@ -72,50 +69,25 @@ struct ActStage {
             v[i] = make_uint4(0, 0, 0, 0);
             ok[i] = true;
             if (off[i] != ~0u && kin) {
-                const char* src = static_cast<const char*>(p.x) + ((size_t)off[i] + k0) * kEsz;
-                {
-                    uint32_t t[4];
-                    if (kEsz == 4) {
+                const uint16_t* s16 = x + (size_t)off[i] + k0;
+                uint32_t t[4];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) t[e] = reinterpret_cast<const uint32_t*>(src)[e];
-                    } else {
-                        const uint16_t* s16 = reinterpret_cast<const uint16_t*>(src);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) t[e] = (uint32_t)s16[2 * e] | ((uint32_t)s16[2 * e + 1] << 16);
-                    }
-                    v[i] = make_uint4(t[0], t[1], t[2], t[3]);
-                }
+                for (int e = 0; e < 4; ++e) t[e] = (uint32_t)s16[2 * e] | ((uint32_t)s16[2 * e + 1] << 16);
+                v[i] = make_uint4(t[0], t[1], t[2], t[3]);
             }
         }
     }
 
-    // hi (and, for fp32 input, lo) tiles [BM][kAPitch] of 16-bit MFMA operands.
-    __device__ __forceinline__ void store(uint16_t* hi, uint16_t* lo) const {
+    // the [BM][kAPitch] tile of MFMA operands
+    __device__ __forceinline__ void store(uint16_t* a) const {
         const int cu = threadIdx.x % kUnitsPerRow, r0 = threadIdx.x / kUnitsPerRow;
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
-            const int off_lds = (r0 + i * kRowsPerPass) * kAPitch + cu * kElems;
             // a mask, not a select: a select of the loaded value lets the compiler branch around the use, and the
             // joins make its wait counts fall back to waiting for every outstanding load
             const uint32_t mk = 0u - (uint32_t)ok[i];
-            const uint4 vi = make_uint4(v[i].x & mk, v[i].y & mk, v[i].z & mk, v[i].w & mk);
-            if (XT != XT_F32) {
-                *reinterpret_cast<uint4*>(hi + off_lds) = vi;
-            } else {
-                const float f[4] = {__builtin_bit_cast(float, vi.x), __builtin_bit_cast(float, vi.y),
-                                    __builtin_bit_cast(float, vi.z), __builtin_bit_cast(float, vi.w)};
-                uint32_t h[2], l[2];
-#pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    const uint16_t h0 = float_to_bf16_bits(f[2 * e]), h1 = float_to_bf16_bits(f[2 * e + 1]);
-                    const uint16_t l0 = float_to_bf16_bits(f[2 * e] - bf16_bits_to_float(h0));
-                    const uint16_t l1 = float_to_bf16_bits(f[2 * e + 1] - bf16_bits_to_float(h1));
-                    h[e] = (uint32_t)h0 | ((uint32_t)h1 << 16);
-                    l[e] = (uint32_t)l0 | ((uint32_t)l1 << 16);
-                }
-                *reinterpret_cast<uint2*>(hi + off_lds) = make_uint2(h[0], h[1]);
-                *reinterpret_cast<uint2*>(lo + off_lds) = make_uint2(l[0], l[1]);
-            }
+            *reinterpret_cast<uint4*>(a + (r0 + i * kRowsPerPass) * kAPitch + cu * kElems) =
+                make_uint4(v[i].x & mk, v[i].y & mk, v[i].z & mk, v[i].w & mk);
         }
     }
 };
@@ -193,29 +165,6 @@ struct Mfma<_Float16> {
     }
 };
 
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-
-// Eight int8 codes (in a uint2) to eight 16-bit operand values: exact codes, or T(fp32(d) * q). Pairs are rounded
-// together (one v_cvt_pk_bf16_f32 for bf16).
-template <typename T, int MODE>
-__device__ __forceinline__ uint4 codes_to_operand(uint2 raw, float d) {
-    typedef typename std::conditional<std::is_same<T, __bf16>::value, bf16x2, f16x2>::type T2;
-    uint32_t out[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const uint32_t word = e < 2 ? raw.x : raw.y;
-        const int sh = 16 * (e & 1);
-        f32x2 f;
-        f.x = (float)(int)(int8_t)(uint8_t)(word >> sh);
-        f.y = (float)(int)(int8_t)(uint8_t)(word >> (sh + 8));
-        if (MODE == MODE_DEQUANT) f = f * d;
-        out[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, T2));
-    }
-    return make_uint4(out[0], out[1], out[2], out[3]);
-}
-
 // Converts the raw [BN][68-byte] stage into 16-bit B operands [BN][kAPitch] (and, for EXACT, fp32 scales [BN][2]).
 // Thread t handles row t / 2 (+128 per pass) and the four 8-code chunks (blk, jj = 2 q + t % 2): block 0's codes sit
 // at byte 2 + 8 jj (two bytes off dword alignment, realigned with alignbyte), block 1's at byte 36 + 8 jj.
@@ -260,117 +209,28 @@ __device__ __forceinline__ void convert_stage(const uint32_t* raw, uint16_t* b, 
     }
 }
 
-// ------------------------------------------------------------------------------------------------ epilogue
-// Epilogue through LDS: the accumulator tile is written to LDS as fp32 ([BM][BN + 4]), then each thread takes runs of
-// 8 consecutive columns of one row and applies the epilogue with vector loads of bias and residual and one 16-byte
-// (32-byte for fp32) store per run, so each wave writes whole row segments instead of 2-byte scattered stores.
-// KS == 2: the workgroup's waves form two depth groups and only the first group's accumulators (which already hold
-// the second group's sums) are written.
-template <int BM, int BN, int TM, int TN, int WM, int WN, int THREADS, int KS = 1>
-__device__ __forceinline__ void write_tile_staged(const GemmParams& p, const f32x16 (&acc)[TM][TN], int m0, int n0,
-                                                  float* stage) {
-    constexpr int kPitch = BN + 4;
-    constexpr int kRuns = BN / 8;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wq = wave % (THREADS / 64 / KS);
-    const int wm = wq >> 1, wn = wq & 1;
-    const bool round_first = (p.flags & IDOLQ_FLAG_ROUND_BEFORE_BIAS) != 0;
-    __syncthreads();
-#pragma unroll
-    for (int tn = 0; tn < TN; ++tn) {
-        if (KS == 2 && wave >= THREADS / 128) break;
-        const int col = wn * WN + tn * 32 + (lane & 31);
-        const float bias = p.bias && n0 + col < p.n ? load_as_float(p.bias, p.bias_dt, n0 + col) : 0.0f;
-#pragma unroll
-        for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = wm * WM + tm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                float v = acc[tm][tn][r];
-                if (round_first) v = round_through(p.y_dt, v);
-                stage[row * kPitch + col] = v + bias;
-            }
-    }
-    __syncthreads();
-    for (int c = threadIdx.x; c < BM * kRuns; c += THREADS) {
-        const int row = c / kRuns, col = (c % kRuns) * 8;
-        const int grow = m0 + row, gcol = n0 + col;
-        if (grow >= p.m || gcol >= p.n) continue;
-        float v[8];
-        const float4 lo = *reinterpret_cast<const float4*>(stage + row * kPitch + col);
-        const float4 hi = *reinterpret_cast<const float4*>(stage + row * kPitch + col + 4);
-        v[0] = lo.x, v[1] = lo.y, v[2] = lo.z, v[3] = lo.w, v[4] = hi.x, v[5] = hi.y, v[6] = hi.z, v[7] = hi.w;
-        const int cnt = min(8, p.n - gcol);
-        if (cnt == 8 && p.y_vec) {
-            float r[8];
-            if (p.res) {
-                const char* rp = static_cast<const char*>(p.res) + ((int64_t)grow * p.ldr + gcol) * (p.res_dt == IDOLQ_F32 ? 4 : 2);
-                if (p.res_dt == IDOLQ_F32) {
-                    const float4 a = reinterpret_cast<const float4*>(rp)[0], b = reinterpret_cast<const float4*>(rp)[1];
-                    r[0] = a.x, r[1] = a.y, r[2] = a.z, r[3] = a.w, r[4] = b.x, r[5] = b.y, r[6] = b.z, r[7] = b.w;
-                } else {
-                    const uint4 u = *reinterpret_cast<const uint4*>(rp);
-                    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const uint16_t bits = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
-                        r[e] = p.res_dt == IDOLQ_BF16 ? bf16_bits_to_float(bits) : half_bits_to_float(bits);
-                    }
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = apply_act(p.act, p.res ? v[e] + r[e] : v[e]);
-            char* yp = static_cast<char*>(p.y) + ((int64_t)grow * p.ldy + gcol) * (p.y_dt == IDOLQ_F32 ? 4 : 2);
-            if (p.y_dt == IDOLQ_F32) {
-                reinterpret_cast<float4*>(yp)[0] = make_float4(v[0], v[1], v[2], v[3]);
-                reinterpret_cast<float4*>(yp)[1] = make_float4(v[4], v[5], v[6], v[7]);
-            } else {
-                uint32_t w[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint16_t a = p.y_dt == IDOLQ_BF16 ? float_to_bf16_bits(v[2 * e]) : float_to_half_bits(v[2 * e]);
-                    const uint16_t b = p.y_dt == IDOLQ_BF16 ? float_to_bf16_bits(v[2 * e + 1]) : float_to_half_bits(v[2 * e + 1]);
-                    w[e] = (uint32_t)a | ((uint32_t)b << 16);
-                }
-                *reinterpret_cast<uint4*>(yp) = make_uint4(w[0], w[1], w[2], w[3]);
-            }
-        } else {
-            for (int e = 0; e < cnt; ++e) {
-                float x = v[e];
-                if (p.res) x += load_as_float(p.res, p.res_dt, (int64_t)grow * p.ldr + gcol + e);
-                store_from_float(p.y, p.y_dt, (int64_t)grow * p.ldy + gcol + e, apply_act(p.act, x));
-            }
-        }
-    }
-}
-
 // ------------------------------------------------------------------------------------------------ 16-bit MFMA kernel
 // Software pipeline with one barrier per stage. At the start of stage s: A[s%2] and B[s%2] hold stage s, raw[(s+1)%2]
 // holds stage s+1's weight bytes, one activation register set holds stage s+1 and one weight register set stage s+2.
 // During stage s each wave stores those registers (A[(s+1)%2], raw[s%2]), reloads them with activations s+3 and
 // weights s+4, converts raw[(s+1)%2] into B[(s+1)%2] and runs the MFMAs of stage s; every buffer it writes was last
 // read in stage s-1, before the barrier that ends it.
-// KS == 2 (EXACT): the waves form two depth groups of (THREADS / 256) x 2; group g multiplies block g of every
-// two-block stage into its own accumulators, and the second group's sums are added to the first's at the end (twice
-// the waves per workgroup for the latency of the per-block MFMA chains, the same loads and conversion).
-template <int BM, int BN, int XT, int MODE, bool W4, int THREADS, int KS = 1, bool XA = false>
+template <int BM, int BN, int XT, int MODE, bool W4, int THREADS>
 __global__ __launch_bounds__(THREADS) void q8_gemm_kernel(GemmParams p) {
     typedef typename std::conditional<XT == XT_F16, _Float16, __bf16>::type T;
     typedef typename Mfma<T>::vec Vec;
-    constexpr int NT = XT == XT_F32 ? 2 : 1;  // activation terms: bf16 high and low parts of fp32 input
-    static_assert(KS == 1 || (KS == 2 && MODE == MODE_EXACT), "depth groups are for the EXACT fold");
-    // waves in a (THREADS / KS / 128) x 2 grid per depth group, each owning a WM x WN tile of 32 x 32 MFMA tiles
-    constexpr int WAVES_M = THREADS / KS / 128;
-    constexpr int NB = 2 / KS;  // blocks of a stage each wave multiplies
+    // waves in a (THREADS / 128) x 2 grid, each owning a WM x WN tile of 32 x 32 MFMA tiles
+    constexpr int WAVES_M = THREADS / 128;
+    constexpr int NB = 2;  // blocks of a stage
     constexpr int WM = BM / WAVES_M, WN = BN / 2, TM = WM / 32, TN = WN / 32;
 
     constexpr int kRawWords = RawStage<BN, W4, THREADS>::kWords;
-    constexpr int kABytes = 2 * NT * BM * kAPitch * 2, kBBytes = 2 * BN * kAPitch * 2, kRawBytes = 2 * kRawWords * 4;
+    constexpr int kABytes = 2 * BM * kAPitch * 2, kBBytes = 2 * BN * kAPitch * 2, kRawBytes = 2 * kRawWords * 4;
     constexpr int kScaleBytes = MODE == MODE_EXACT ? 2 * BN * 2 * 4 : 16;
     constexpr int kLoopBytes = kABytes + kBBytes + kRawBytes + kScaleBytes;
     constexpr int kStageBytes = BM * (BN + 4) * 4;
     __shared__ __attribute__((aligned(16))) char smem[kLoopBytes > kStageBytes ? kLoopBytes : kStageBytes];
-    typedef uint16_t ATile[NT][BM * kAPitch];
+    typedef uint16_t ATile[BM * kAPitch];
     typedef uint16_t BTile[BN * kAPitch];
     typedef uint32_t RawTile[kRawWords];
     typedef float ScaleTile[MODE == MODE_EXACT ? BN * 2 : 4];
@@ -380,9 +240,7 @@ __global__ __launch_bounds__(THREADS) void q8_gemm_kernel(GemmParams p) {
     ScaleTile* bscale = reinterpret_cast<ScaleTile*>(smem + kABytes + kBBytes + kRawBytes);
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int kg = KS == 2 ? wave / (THREADS / 128) : 0;  // depth group
-    const int wq = wave % (THREADS / 64 / KS);
-    const int wm = wq >> 1, wn = wq & 1;
+    const int wm = wave >> 1, wn = wave & 1;
     int tile_m, tile_n;
     tile_coords(p.tiles_m, p.tiles_n, tile_m, tile_n);
     const int m0 = tile_m * BM, n0 = tile_n * BN;
@@ -400,7 +258,7 @@ __global__ __launch_bounds__(THREADS) void q8_gemm_kernel(GemmParams p) {
     // Two register sets for the activation and weight loads, used alternately, so every load is issued two stages
     // before its registers are stored to LDS: set (s + 1) % 2 of activations holds stage s + 1 at the start of
     // stage s, set s % 2 of weights holds stage s + 2.
-    ActStage<BM, XT, THREADS, XA> as0, as1;
+    ActStage<BM, THREADS> as0, as1;
     RawStage<BN, W4, THREADS> ws0, ws1;
     as0.init(p, m0);
     as1.init(p, m0);
@@ -415,7 +273,7 @@ __global__ __launch_bounds__(THREADS) void q8_gemm_kernel(GemmParams p) {
         as1.load(p, kKStep);
         ws1.load(p, 2, nblocks);
     }
-    as0.store(a_lds[0][0], a_lds[0][NT - 1]);
+    as0.store(a_lds[0]);
     ws0.store(raw_lds[0]);
     if (nsteps > 2) {
         as0.load(p, 2 * kKStep);
@@ -431,7 +289,7 @@ __global__ __launch_bounds__(THREADS) void q8_gemm_kernel(GemmParams p) {
         // The body has no branches: past the last stage the prefetch indices are clamped and the stores and the
         // conversion fill buffers that are never read again, so the whole stage is one scheduling region.
         const int cur = s & 1, nxt = cur ^ 1;
-        ra.store(a_lds[nxt][0], a_lds[nxt][NT - 1]);
+        ra.store(a_lds[nxt]);
         ra.load(p, min(s + 3, nsteps - 1) * kKStep);
         rw.store(raw_lds[cur]);
         rw.load(p, 2 * min(s + 4, nsteps - 1), nblocks);
@@ -440,41 +298,35 @@ __global__ __launch_bounds__(THREADS) void q8_gemm_kernel(GemmParams p) {
         const uint16_t* bc = b_lds[cur];
         // Operands of the wave's blocks of the stage are read before the first MFMA (the second block's reads
         // complete under the first block's MFMAs).
-        Vec a[NB][NT][TM][2], b[NB][TN][2];
+        Vec a[NB][TM][2], b[NB][TN][2];
 #pragma unroll
         for (int bi = 0; bi < NB; ++bi)
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const int koff = (KS == 2 ? kg : bi) * 32 + h * 16 + (lane >> 5) * 8;
+                const int koff = bi * 32 + h * 16 + (lane >> 5) * 8;
 #pragma unroll
-                for (int t = 0; t < NT; ++t)
-#pragma unroll
-                    for (int tm = 0; tm < TM; ++tm)
-                        a[bi][t][tm][h] = *reinterpret_cast<const Vec*>(a_lds[cur][t] + (wm * WM + tm * 32 + (lane & 31)) * kAPitch + koff);
+                for (int tm = 0; tm < TM; ++tm)
+                    a[bi][tm][h] = *reinterpret_cast<const Vec*>(a_lds[cur] + (wm * WM + tm * 32 + (lane & 31)) * kAPitch + koff);
 #pragma unroll
                 for (int tn = 0; tn < TN; ++tn)
                     b[bi][tn][h] = *reinterpret_cast<const Vec*>(bc + (wn * WN + tn * 32 + (lane & 31)) * kAPitch + koff);
             }
 #pragma unroll
         for (int bi = 0; bi < NB; ++bi) {
-            const int blk = KS == 2 ? kg : bi;
 #pragma unroll
             for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
                 for (int tn = 0; tn < TN; ++tn) {
                     if (MODE == MODE_DEQUANT) {
-                        acc[tm][tn] = Mfma<T>::run(a[bi][0][tm][0], b[bi][tn][0], acc[tm][tn]);
-                        acc[tm][tn] = Mfma<T>::run(a[bi][0][tm][1], b[bi][tn][1], acc[tm][tn]);
+                        acc[tm][tn] = Mfma<T>::run(a[bi][tm][0], b[bi][tn][0], acc[tm][tn]);
+                        acc[tm][tn] = Mfma<T>::run(a[bi][tm][1], b[bi][tn][1], acc[tm][tn]);
                     } else {
-                        const float d = bscale[cur][(wn * WN + tn * 32 + (lane & 31)) * 2 + blk];
+                        const float d = bscale[cur][(wn * WN + tn * 32 + (lane & 31)) * 2 + bi];
                         f32x16 part;
 #pragma unroll
                         for (int r = 0; r < 16; ++r) part[r] = 0.0f;
-#pragma unroll
-                        for (int t = 0; t < NT; ++t) {
-                            part = Mfma<T>::run(a[bi][t][tm][0], b[bi][tn][0], part);
-                            part = Mfma<T>::run(a[bi][t][tm][1], b[bi][tn][1], part);
-                        }
+                        part = Mfma<T>::run(a[bi][tm][0], b[bi][tn][0], part);
+                        part = Mfma<T>::run(a[bi][tm][1], b[bi][tn][1], part);
 #pragma unroll
                         for (int r = 0; r < 16; ++r) acc[tm][tn][r] = fmaf(part[r], d, acc[tm][tn][r]);
                     }
@@ -487,32 +339,7 @@ __global__ __launch_bounds__(THREADS) void q8_gemm_kernel(GemmParams p) {
         stage(s, as1, ws0);
         if (s + 1 < nsteps) stage(s + 1, as0, ws1);
     }
-    if constexpr (KS == 2) {
-        // the second group's sums (odd blocks) through LDS into the first group's (even blocks): a fixed order
-        float* red = reinterpret_cast<float*>(smem);
-        constexpr int kPitch = BN + 4;
-        __syncthreads();
-        if (kg == 1)
-#pragma unroll
-            for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-                for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        red[(wm * WM + tm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * kPitch + wn * WN + tn * 32 +
-                            (lane & 31)] = acc[tm][tn][r];
-        __syncthreads();
-        if (kg == 0)
-#pragma unroll
-            for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-                for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        acc[tm][tn][r] += red[(wm * WM + tm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * kPitch +
-                                              wn * WN + tn * 32 + (lane & 31)];
-    }
-    write_tile_staged<BM, BN, TM, TN, WM, WN, THREADS, KS>(p, acc, m0, n0, reinterpret_cast<float*>(smem));
+    write_tile_staged<BM, BN, TM, TN, WM, WN, THREADS>(p, acc, m0, n0, reinterpret_cast<float*>(smem));
 }
 
 // ------------------------------------------------------------------------------------------------ launch
@@ -532,52 +359,8 @@ int launch_16bit_tile(GemmParams p, int xt, int mode, bool w4, hipStream_t strea
     return check_launch("q8_gemm_kernel");
 }
 
-// fp32 activations (EXACT): eight waves in two depth groups (the even and the odd block of each stage)
-template <int BM, int BN>
-int launch_f32_tile(GemmParams p, bool w4, hipStream_t stream) {
-    p.tiles_m = (p.m + BM - 1) / BM;
-    p.tiles_n = (p.n + BN - 1) / BN;
-    const dim3 grid(p.tiles_m * p.tiles_n), block(2 * kThreads);
-    if (w4 && p.x_aligned)
-        hipLaunchKernelGGL((q8_gemm_kernel<BM, BN, XT_F32, MODE_EXACT, true, 2 * kThreads, 2, true>), grid, block, 0, stream, p);
-    else if (w4)
-        hipLaunchKernelGGL((q8_gemm_kernel<BM, BN, XT_F32, MODE_EXACT, true, 2 * kThreads, 2>), grid, block, 0, stream, p);
-    else
-        hipLaunchKernelGGL((q8_gemm_kernel<BM, BN, XT_F32, MODE_EXACT, false, 2 * kThreads, 2>), grid, block, 0, stream, p);
-    return check_launch("q8_gemm_kernel");
-}
-
-// Tile choice: one workgroup per CU fits in LDS, so a launch runs in ceil(tiles / 256) rounds on the 256 CUs; pick
-// the tile with the smallest rounds * tile area / efficiency (the per-CU critical path). `eff` is the tile's measured
-// throughput relative to the 256 x 128 eight-wave tile on a large GEMM (4096 x 6144 x 1536).
-struct TileChoice {
-    int bm, bn;
-    float eff;
-};
-
-TileChoice choose_tile(int m, int n, const TileChoice* cands, int count) {
-    constexpr long kCUs = 256;
-    TileChoice best = cands[0];
-    float best_cost = -1.0f;
-    for (int i = 0; i < count; ++i) {
-        const long tiles = (long)((m + cands[i].bm - 1) / cands[i].bm) * ((n + cands[i].bn - 1) / cands[i].bn);
-        const float cost = (float)((tiles + kCUs - 1) / kCUs * cands[i].bm * cands[i].bn) / cands[i].eff;
-        if (best_cost < 0.0f || cost < best_cost) {
-            best = cands[i];
-            best_cost = cost;
-        }
-    }
-    return best;
-}
-
 int launch_16bit(GemmParams p, int xt, int mode, bool w4, void* workspace, size_t workspace_bytes, hipStream_t stream) {
-    if (xt == XT_F32) {
-        static const TileChoice cands[] = {{128, 128, 1.0f}, {128, 64, 1.0f}, {64, 64, 0.75f}};
-        const TileChoice t = choose_tile(p.m, p.n, cands, 3);
-        if (t.bn == 128) return launch_f32_tile<128, 128>(p, w4, stream);
-        if (t.bm == 128) return launch_f32_tile<128, 64>(p, w4, stream);
-        return launch_f32_tile<64, 64>(p, w4, stream);
-    }
+    if (xt == XT_F32) return launch_exact_rows(p, w4, stream);
     static const TileChoice cands[] = {{256, 128, 1.0f}, {128, 128, 0.5f}, {128, 64, 0.6f}};
     const TileChoice t = choose_tile(p.m, p.n, cands, 3);
     if (p.w_tiled) {

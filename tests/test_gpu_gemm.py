@@ -117,6 +117,26 @@ def test_int8_row_major_tiles_fold_block_by_block(m, n, k, skew):
     assert norm_rel(got, xs @ ws.T) < 1e-6
 
 
+@pytest.mark.parametrize("m,n,k", [(17, 33, 64), (64, 64, 512), (65, 63, 576), (100, 130, 4032), (40, 96, 96),
+                                   (1100, 2100, 160), (1100, 4100, 128), (300, 4096, 192)])
+@pytest.mark.parametrize("xskew,wskew", [(0, 0), (1, 0), (0, 2)])
+def test_exact_row_major_tiles_with_fp32_rows(m, n, k, xskew, wskew):
+    # the EXACT kernels of fp32 rows on row-major weights: the 64 x 64 tile split over the depth (one pair of blocks, a
+    # pair per wave, one more), the 64 x 64, 128 x 64 and 128 x 128 tiles, partial tiles, last stages of fewer blocks,
+    # x rows off 16 bytes and weight rows off a dword. x in 16 bits (two bf16 parts, 2^-17 of a value at most): 1e-5
+    rng = np.random.default_rng(m + n + k)
+    a = rng.normal(0, 1, (m, k + 1)).astype(np.float32)
+    w, bias = q8(rng, n, k, 0.05), rng.normal(0, 0.01, n).astype(np.float32)
+    x = to_dev(a)[:, 1:] if xskew else to_dev(np.ascontiguousarray(a[:, 1:]))
+    buf = torch.zeros(w.size + wskew, dtype=torch.uint8, device=DEV)
+    buf[wskew:] = to_dev(w.reshape(-1))
+    got = L.gemm(x, buf[wskew:], n, bias=to_dev(bias), mode=L.MODE_EXACT, out_dtype=torch.float32).cpu().numpy()
+    blocks = w.reshape(n, k // 32, 34)
+    d = np.ascontiguousarray(blocks[:, :, :2]).view(np.float16)[:, :, 0].astype(np.float64)
+    ws = (blocks[:, :, 2:].view(np.int8) * d[:, :, None]).reshape(n, k)
+    assert norm_rel(got, a[:, 1:].astype(np.float64) @ ws.T + bias) < 1e-5
+
+
 def test_gemm_against_reference_golden_vectors(golden):
     # The reference's own outputs for its test shapes (tests/golden/gemm_q8.npz): EXACT vs the float kernel and INT8
     # vs the integer kernel, fp32 in and out, each within 1e-5 norm-relative, on row-major Q8_0 blocks and (five of
