@@ -381,6 +381,7 @@ def _attention_workspace(device, nbytes):
 _attention_workspaces = {}
 
 
+F32_WHOLE_KEYS = 128  # up to four 32-key tiles a key range is never cut (the merge alone costs more than they do)
 STAGED_V_MIN_KEYS = 2048  # measured: staging V pays from about 32 key tiles (its launch costs ~5 us)
 
 
@@ -395,7 +396,7 @@ def attention(q, k, v, batch, lq, lk, heads, head_dim, ldq, ldkv, q_bs, kv_bs, o
         raise ValueError("q, k and v must share a dtype")
     if q.dtype == torch.float32:
         # the parts of a cut key range: from the allocator's stream-ordered pool for this call alone
-        need = int(lib.idolq_attention_f32_workspace(batch, lq, lk, heads, head_dim))
+        need = int(lib.idolq_attention_f32_workspace(batch, lq, lk, heads, head_dim)) if lk > F32_WHOLE_KEYS else 0
         ws = torch.empty(need, device=q.device, dtype=torch.uint8) if need else None
     else:
         if staged_v is None:
