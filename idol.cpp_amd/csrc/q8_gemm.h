@@ -65,6 +65,10 @@ bool wide_eligible(const GemmParams& p, int xt, int mode);
 size_t wide_workspace_bytes();
 constexpr size_t kWideCountBytes = 4096;  // the tile counters at the start of that workspace (zero between launches)
 int launch_wide(GemmParams p, int xt, void* workspace, size_t workspace_bytes, hipStream_t stream);
+// The grouped-layout kernel's small tiles (q8_gemm_wide_small.hip): 32 rt x 128, rt = 1 or 2, whole tiles; set_y_vec4
+// has been called on p. The number of its workgroups that share a CU.
+int launch_wide_small(const GemmParams& p, int xt, bool q4k, int rt, hipStream_t stream);
+int wide_small_slots(int rt);
 // The INT8 mode on tiled weights (p.qa, p.sa from the tiled quantizer); workspace as launch_wide's (may be null).
 int launch_wide_i8(GemmParams p, void* workspace, size_t workspace_bytes, hipStream_t stream);
 // The EXACT mode on tiled weights (p.x, p.x_lo: bf16 high and low parts of the activations, row stride k).

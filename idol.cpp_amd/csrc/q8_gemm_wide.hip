@@ -86,13 +86,24 @@ GemmParams column_window(GemmParams p, int n0, int n) {
 //   128-row tiles with stream-K over the tiles left after the whole rounds (a workspace is needed; about 6 more for
 //     the partial tiles). 256-row tiles are not split: on the MLP block's down projection (4096 x 6144 -> 1536) their
 //     stream-K plan took 134 us against 105 us for 128-row stream-K; the split ranges lose the L2 sharing of
-//     neighbouring workgroups.
+//     neighbouring workgroups;
+//   small tiles (32 or 64 x 128, q8_gemm_wide_small.hip), several of them on a CU, where the others leave CUs idle: a
+//     64-deep stage takes STAGE alone on a CU and MORE for each further tile there. Bit-identical, us (best larger
+//     tile against the small tile taken): 64 x 4096 x 1024 17.7 against 8.6, 64 x 1024 x 4096 54 against 27, 333 x 4608
+//     x 1536 25.1 against 14.9 (Q4_K 31.7 against 19.1), 1000 x 1536 x 1536 24.7 against 14.6, 1000 x 4608 x 1536 27.7
+//     against 26.5; from about two rounds on the larger tiles win (2000 x 6144 x 1536 43 against 55).
 struct WideShape {
     int rt, ct;
     double stage, fixed;
 };
 constexpr WideShape kShapes[3] = {{8, 2, 1.42, 16.0}, {4, 2, 0.85, 9.0}, {4, 3, 1.16, 12.0}};
 constexpr int kNumShapes = sizeof(kShapes) / sizeof(kShapes[0]);
+
+struct SmallShape {
+    int rt;
+    double stage, more, fixed;
+};
+constexpr SmallShape kSmallShapes[2] = {{1, 0.445, 0.31, 2.9}, {2, 0.50, 0.30, 3.6}};
 
 template <typename T, bool Q4K, int RT, int CT>
 int launch_shape(GemmParams p, const WideSplit& sp, bool split, hipStream_t stream) {
@@ -132,6 +143,16 @@ int launch_wide_dtype(GemmParams p, void* workspace, size_t workspace_bytes, hip
     const double hybrid = cb8 > 0 && cb8 < tn ? rounds(tm8 * cb8) * (S * c8.stage + c8.fixed) +
                                                     rounds(tm4 * (tn - cb8)) * (S * c4.stage + c4.fixed)
                                               : -1.0;
+    int small = 0;
+    double small_cost = 0.0;
+    for (const SmallShape& c : kSmallShapes) {
+        const long tiles = (long)((p.m + 32 * c.rt - 1) / (32 * c.rt)) * ((p.n + 127) / 128), slots = wide_small_slots(c.rt);
+        auto round = [&](long on_cu) { return on_cu == 0 ? 0.0 : S * (c.stage + c.more * (on_cu - 1)) + c.fixed; };
+        const double cost = tiles / (cus * slots) * round(slots) + round((tiles % (cus * slots) + cus - 1) / cus);
+        if (!small || cost < small_cost) small = c.rt, small_cost = cost;
+    }
+    if (small_cost < best && (hybrid < 0 || small_cost < hybrid))
+        return launch_wide_small(p, std::is_same<T, __bf16>::value ? XT_BF16 : XT_F16, Q4K, small, stream);
     const WideSplit none{0, 0, 0, 0, nullptr, nullptr};
     auto whole = [&](long tiles) { WideSplit sp = none; sp.G = (int)std::min(tiles, cus); return sp; };
     if (hybrid > 0 && hybrid < best) {

@@ -87,9 +87,12 @@ struct WideSplit {
 // rows x 64 int8 codes, then the rows' two fp32 block scales), kFoldExact (the EXACT mode: BM rows x 64 bf16 high
 // parts, then BM rows x 64 bf16 low parts of fp32 activations).
 constexpr int kFoldI8 = 1, kFoldExact = 2;
-// workgroups per CU of each mode's kernel (its launch bounds; the INT8 fold runs two, see q8_gemm_wide_fold.hip)
+// workgroups per CU of each mode's kernel (its launch bounds; the INT8 fold runs two, see q8_gemm_wide_fold.hip; the
+// small tiles of q8_gemm_wide_small.hip as many as their LDS allows)
 template <int FOLD>
 constexpr int kWideFoldSlots = FOLD == kFoldI8 ? 2 : 1;
+template <int RT, int CT, int FOLD>
+constexpr int kWideSlots = RT * CT >= 8 ? kWideFoldSlots<FOLD> : RT == 2 ? 3 : 4;
 template <int RT, int CT, bool Q4K = false, int FOLD = 0>
 struct WideCfg {
     static constexpr bool I8 = FOLD == kFoldI8, EX = FOLD == kFoldExact;
@@ -321,9 +324,12 @@ __device__ __forceinline__ void wide_tiles(const GemmParams& p, const WideSplit&
     // VALU work stays within the 32 cycles of its MFMA: in steps 0..2 piece q goes after MFMA PS q + PS - 1; in step 3,
     // whose pieces convert the next stage's codes read from LDS in its first slots, the pieces fill the second half
     // (FC on), PF per slot.
-    constexpr int PS = NM / NP;
-    constexpr int FC = NM / 2, PF = NP / (NM - FC);
-    static_assert(NM % NP == 0 && NP % (NM - FC) == 0, "conversion slots");
+    // SM: tiles of fewer than 8 MFMAs a step (q8_gemm_wide_small.hip) have too few slots for this and take whole stages
+    // at a time (below).
+    constexpr bool SM = NM < 8;
+    constexpr int PS = SM ? 1 : NM / NP;
+    constexpr int FC = NM / 2, PF = SM ? 1 : NP / (NM - FC);
+    static_assert(SM || (NM % NP == 0 && NP % (NM - FC) == 0), "conversion slots");
     // One 16-deep step: MFMA i on operand set `cur`, then slot(i) -- the other work of the stage (loads, the next
     // step's LDS reads and conversion) -- each slot pinned after its MFMA by a scheduling barrier, so that this work
     // is issued while the matrix core runs the step instead of being moved next to its first use.
@@ -370,6 +376,75 @@ __device__ __forceinline__ void wide_tiles(const GemmParams& p, const WideSplit&
                 for (int q = 0; q < PF; ++q) convert_piece(0, 0, (i - FC) * PF + q);
             }
         });
+    };
+
+    // SM: the operands of a whole stage in registers, two sets. After the barrier that publishes stage s + 1 its x
+    // operands and weight bytes are read and converted while the MFMAs of stage s run (one scheduling region): per stage
+    // the chain is one barrier, one LDS round trip and the conversion instead of one round trip per 16-deep step. The
+    // loads are issued and waited for in the order of the loop above (n stages, those of stage 0 published).
+    auto small_stages = [&](int n) __attribute__((always_inline)) {
+        Vec sx[2][4][RT];
+        uint4 sw[2][4][CT];
+        auto fetch = [&](int stage, auto set) __attribute__((always_inline)) {
+            constexpr int q = decltype(set)::value;
+            const int buf = stage % 3;
+#pragma unroll
+            for (int c = 0; c <= CT; ++c) read_raw_piece(buf, c, stage);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+                    sx[q][j][rt] = *reinterpret_cast<const Vec*>(smem + buf * C::ABuf + x_lane[j] + rt * 4096);
+        };
+        auto convert = [&](auto set) __attribute__((always_inline)) {
+            constexpr int q = decltype(set)::value;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+#pragma unroll
+                for (int e = 0; e < NP; ++e) convert_piece(j, 0, e);
+#pragma unroll
+                for (int c = 0; c < CT; ++c) sw[q][j][c] = wq[0][c];
+            }
+        };
+        auto multiply = [&](auto set) __attribute__((always_inline)) {
+            constexpr int q = decltype(set)::value;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < NM; ++i)
+                    acc[i / CT][i % CT] = PipeMfma<T>::run(__builtin_bit_cast(Vec, sw[q][j][i % CT]), sx[q][j][i / CT],
+                                                           acc[i / CT][i % CT]);
+        };
+        auto stage = [&](int s, auto set) __attribute__((always_inline)) {
+            constexpr int q = decltype(set)::value;
+            const std::integral_constant<int, q ^ 1> other;
+            if (s + 2 < n) {
+                issue_w(s + 2);
+                wait_vm<DA + DW>();  // W(s + 1) and A(s + 1): A(s + 2), W(s + 2) may remain
+            } else {
+                wait_vm<0>();
+            }
+            __syncthreads();
+            if (s + 3 < n) issue_a(s + 3);
+            fetch(s + 1, other);
+            multiply(set);
+            convert(other);
+        };
+        const std::integral_constant<int, 0> s0;
+        const std::integral_constant<int, 1> s1;
+        fetch(0, s0);
+        convert(s0);
+        int s = 0;
+        for (; s + 2 < n; s += 2) {
+            stage(s, s0);
+            stage(s + 1, s1);
+        }
+        if (s + 1 < n) {
+            stage(s, s0);
+            multiply(s1);
+        } else {
+            multiply(s0);
+        }
     };
 
     // ---- epilogue
@@ -739,6 +814,10 @@ __device__ __forceinline__ void wide_tiles(const GemmParams& p, const WideSplit&
         else
             wait_vm<0>();
         __syncthreads();
+        if constexpr (SM) {
+            small_stages(S);
+            return;
+        }
 #pragma unroll
         for (int c = 0; c <= CT; ++c) read_raw_piece(0, c, 0);
 #pragma unroll
@@ -912,7 +991,7 @@ __device__ __forceinline__ void wide_tiles(const GemmParams& p, const WideSplit&
 }
 
 template <typename T, int RT, int CT, int ACT, bool FAST, bool RES, bool SPLIT, bool Q4K = false, int FOLD = 0>
-__global__ __launch_bounds__(kWideThreads, kWideFoldSlots<FOLD>) void q8_wide_kernel(GemmParams p, WideSplit sp) {
+__global__ __launch_bounds__(kWideThreads, (kWideSlots<RT, CT, FOLD>)) void q8_wide_kernel(GemmParams p, WideSplit sp) {
     __shared__ __attribute__((aligned(1024))) char smem[WideCfg<RT, CT, Q4K, FOLD>::Lds];
     wide_tiles<T, RT, CT, ACT, FAST, RES, SPLIT, Q4K, FOLD>(p, sp, smem);
 }

@@ -130,6 +130,17 @@ def test_q4_k_gemm_multiplies_the_decoded_weights(m, n_total, k, off, cnt, split
     assert torch.equal(y, again)
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 130, 256), (33, 96, 512), (64, 257, 768), (200, 1100, 1024)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_q4_k_gemm_small_tiles(m, n, k, dtype):
+    # 32 x 128 and 64 x 128 tiles on super-blocks, partial rows and columns, 4 to 16 stages: 1e-5 of the fp32 product
+    w = torch.from_numpy(q4k_blocks(n, k, m + n)).to(DEV)
+    x = torch.from_numpy(np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)).to(DEV).to(dtype)
+    y = L.q4_k_gemm(x, w, n, out_dtype=torch.float32)
+    ref = x.double() @ L.blocks_dequant(w, L.KIND_Q4_K, n, k, dtype).double().t().contiguous()
+    assert norm_rel(y.cpu().numpy(), ref.cpu().numpy()) < 1e-5
+
+
 def test_q4_k_gemm_epilogue_and_fused_rounding():
     # bias, residual aliasing y, tanh-GELU in the register epilogue (bf16 out) against the same steps in fp32 on the
     # expanded weights; and the fused path's order: product rounded to bf16, then the bias

@@ -137,6 +137,26 @@ def test_exact_row_major_tiles_with_fp32_rows(m, n, k, xskew, wskew):
     assert norm_rel(got, a[:, 1:].astype(np.float64) @ ws.T + bias) < 1e-5
 
 
+@pytest.mark.parametrize("m,n,k,off,cnt", [(17, 96, 64, 0, 96), (32, 128, 128, 0, 128), (33, 160, 192, 32, 128),
+                                           (64, 300, 320, 0, 300), (65, 129, 1024, 0, 129), (333, 4608, 256, 0, 4608),
+                                           (700, 2560, 448, 512, 2000), (128, 31, 384, 0, 31)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_small_tiles_give_the_row_major_bits(m, n, k, off, cnt, dtype):
+    # calls of few tiles on tiled weights take 32 x 128 or 64 x 128 tiles (1 to 16 stages, partial rows and columns, up
+    # to several tiles a workgroup): the products and their order are the row-major kernel's, so the bits are
+    rng = np.random.default_rng(m + n + k)
+    x = to_dev(rng.normal(0, 1, (m, k)).astype(np.float32)).to(dtype)
+    w = to_dev(q8(rng, n, k, 0.05))
+    b = to_dev(rng.normal(0, 0.1, n).astype(np.float32))
+    res = to_dev(rng.normal(0, 1, (m, cnt)).astype(np.float32)).to(dtype)
+    wt = L.tile_q8_0(w, n, k)
+    for kw in (dict(bias=b), dict(bias=b, residual=res, act=L.ACT_GELU_TANH), dict(out_dtype=torch.float32),
+               dict(bias=b, flags=L.FLAG_ROUND_BEFORE_BIAS, act=L.ACT_RELU), dict(bias=b, act=L.ACT_SILU)):
+        raw = L.gemm(x, w, n, off, cnt, mode=L.MODE_DEQUANT, **kw)
+        til = L.gemm(x, wt, n, off, cnt, mode=L.MODE_DEQUANT, tiled=True, **kw)
+        assert torch.equal(raw, til), kw
+
+
 def test_gemm_against_reference_golden_vectors(golden):
     # The reference's own outputs for its test shapes (tests/golden/gemm_q8.npz): EXACT vs the float kernel and INT8
     # vs the integer kernel, fp32 in and out, each within 1e-5 norm-relative, on row-major Q8_0 blocks and (five of
