@@ -42,7 +42,7 @@ int launch_wide_pair(GemmParams pa, GemmParams pb, int grid, hipStream_t stream,
     const GemmParams& p = pa;  // both ranges share dtypes, activation and alignment
     const bool fast = p.y_vec4 && pa.n % 4 == 0 && pb.n % 4 == 0 && below_2gb(pa) && below_2gb(pb) && p.y_dt == kYdt &&
                       (!p.res || p.res_dt == kYdt) &&
-                      (!p.bias || p.bias_dt == IDOLQ_F32) &&
+                      (!p.bias || p.bias_dt == IDOLQ_F32 || p.bias_dt == kYdt) &&
                       (p.act == IDOLQ_ACT_NONE || p.act == IDOLQ_ACT_GELU_TANH || p.act == IDOLQ_ACT_RELU);
     const dim3 g(grid), block(kWideThreads);
     if (!fast)

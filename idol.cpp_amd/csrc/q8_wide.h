@@ -452,7 +452,7 @@ __device__ __forceinline__ void wide_tiles(const GemmParams& p, const WideSplit&
     // the activation buffers, free once every wave has finished the last stage), and come back row-major: LPR lanes
     // per row, 4 columns each, so that the residual loads and the output stores move whole rows of the wave's 32 CT
     // columns (every cache line written whole) instead of 8-byte pieces of 32 rows.
-    // FAST (chosen by the host): y and the residual have the activation dtype, the bias is fp32, n is a multiple of 4
+    // FAST (chosen by the host): y and the residual have the activation dtype, the bias is fp32 or that, n is a multiple of 4
     // with vector-aligned 4-column groups, and the activation is ACT; rows and 4-column groups outside y are skipped.
     // Otherwise the general path: per element bounds checks and dtype conversions.
     const bool round_first = (p.flags & IDOLQ_FLAG_ROUND_BEFORE_BIAS) != 0;
@@ -536,9 +536,20 @@ __device__ __forceinline__ void wide_tiles(const GemmParams& p, const WideSplit&
         const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(p.y, 0, 0x7fffffff, kRaw);
         const __amdgpu_buffer_rsrc_t rr =
             __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.res ? p.res : p.y), 0, p.res ? 0x7fffffff : 0, kRaw);
-        const __amdgpu_buffer_rsrc_t rb =
-            __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.bias ? p.bias : p.y), 0, p.bias ? 0x7fffffff : 0, kRaw);
-        const f32x4 b = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, col_ok ? (uint32_t)col * 4 : kOff, 0, 0));
+        // the bias is fp32 or T: a buffer for each, the other one of no bytes, whose loads read the 0 that is added
+        const bool b32 = p.bias_dt == IDOLQ_F32;
+        const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.bias ? p.bias : p.y), 0,
+                                                                            p.bias && b32 ? 0x7fffffff : 0, kRaw);
+        const __amdgpu_buffer_rsrc_t rbt = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.bias ? p.bias : p.y), 0,
+                                                                             p.bias && !b32 ? 0x7fffffff : 0, kRaw);
+        auto bias4 = [&](int c0, bool ok) __attribute__((always_inline)) {
+            const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, ok ? (uint32_t)c0 * 4 : kOff, 0, 0));
+            const auto w = __builtin_amdgcn_raw_buffer_load_b64(rbt, ok ? (uint32_t)c0 * 2 : kOff, 0, 0);
+            const f32x2 lo = __builtin_convertvector(__builtin_bit_cast(T2, (uint32_t)w[0]), f32x2);
+            const f32x2 hi = __builtin_convertvector(__builtin_bit_cast(T2, (uint32_t)w[1]), f32x2);
+            return f32x4{v[0] + lo.x, v[1] + lo.y, v[2] + hi.x, v[3] + hi.y};
+        };
+        const f32x4 b = bias4(col, col_ok);
         f32x4 bacc[CT][4];  // !RES: the biases in the accumulator layout (stage_chunk_act)
         if constexpr (!RES) {
 #pragma unroll
@@ -546,8 +557,7 @@ __device__ __forceinline__ void wide_tiles(const GemmParams& p, const WideSplit&
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const int ca = n0 + wave * 32 * CT + 32 * c + 8 * g + 4 * (lane >> 5);
-                    bacc[c][g] = __builtin_bit_cast(
-                        f32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, ca < p.n ? (uint32_t)ca * 4 : kOff, 0, 0));
+                    bacc[c][g] = bias4(ca, ca < p.n);
                 }
         }
         auto out_off = [&](int row, int64_t ld) __attribute__((always_inline)) {
@@ -1027,7 +1037,7 @@ int launch_wide_s(GemmParams p, const WideSplit& sp, hipStream_t stream) {
     p.tiles_n = (p.n + 128 * CT - 1) / (128 * CT);
     constexpr int kYdt = std::is_same<T, __bf16>::value ? IDOLQ_BF16 : IDOLQ_F16;
     const bool fast = p.y_vec4 && p.n % 4 == 0 && below_2gb(p) && p.y_dt == kYdt && (!p.res || p.res_dt == kYdt) &&
-                      (!p.bias || p.bias_dt == IDOLQ_F32) &&
+                      (!p.bias || p.bias_dt == IDOLQ_F32 || p.bias_dt == kYdt) &&
                       (p.act == IDOLQ_ACT_NONE || p.act == IDOLQ_ACT_GELU_TANH || p.act == IDOLQ_ACT_RELU);
     if (!fast)
         hipLaunchKernelGGL((q8_wide_kernel<T, RT, CT, IDOLQ_ACT_NONE, false, false, SPLIT, Q4K, FOLD>), grid, block, 0, stream,

@@ -49,12 +49,15 @@ def fused_linear(value, packed, shape, kind, bias=None, *, q8_blocks=None, q8_ti
     if not m:
         return torch.empty((*value.shape[:-1], n), device=value.device, dtype=value.dtype)
     w = packed.reshape(-1)
-    # the bias enters the epilogue as fp32, as the reference loads it (an exact widening)
-    b32 = bias.float() if bias is not None else None
+    # The bias enters the epilogue as fp32, as the reference loads it (an exact widening): the small-m, tiled and Q4_K
+    # kernels widen it themselves where its entries are whole vectors; the other row-major kernels take fp32.
+    whole = bias is None or (bias.is_contiguous() and bias.data_ptr() % 16 == 0)
     if kind == KIND_Q4_K:
+        if not whole:
+            bias = bias.float()
         if x.data_ptr() % 16:  # the Q4_K kernel reads 16-byte aligned rows (k % 256 == 0): only a view can miss it
             x = x.clone()
-        out = L.q4_k_gemm(x, w, n, bias=b32, flags=L.FLAG_ROUND_BEFORE_BIAS)
+        out = L.q4_k_gemm(x, w, n, bias=bias, flags=L.FLAG_ROUND_BEFORE_BIAS)
         return out.reshape(*value.shape[:-1], n)
     # the reference's F.linear branch adds the bias before its one rounding; everywhere else the product is rounded
     # first
@@ -62,10 +65,13 @@ def fused_linear(value, packed, shape, kind, bias=None, *, q8_blocks=None, q8_ti
     flags = 0 if dense_branch else L.FLAG_ROUND_BEFORE_BIAS
     # the tiled-weight GEMM reads 16-byte aligned activation rows; other views keep the row-major blocks
     aligned = x.data_ptr() % 16 == 0 and (m == 1 or (x.stride(0) * x.element_size()) % 16 == 0)
-    if q8_tiled is not None and m > SMALL_M and aligned:
+    tiled = q8_tiled is not None and m > SMALL_M and aligned
+    if not (whole and (tiled or (m <= SMALL_M and k % 256 == 0))):
+        bias = bias.float() if bias is not None else None
+    if tiled:
         if q8_tiled.numel() != L.tiled_q8_0_bytes(n, k) or q8_tiled.device != value.device:
             raise ValueError('invalid packed linear dimensions')
-        out = L.gemm(x, q8_tiled.reshape(-1), n, bias=b32, mode=L.MODE_DEQUANT, flags=flags, tiled=True)
+        out = L.gemm(x, q8_tiled.reshape(-1), n, bias=bias, mode=L.MODE_DEQUANT, flags=flags, tiled=True)
         return out.reshape(*value.shape[:-1], n)
     if kind == KIND_Q4_0:
         if q8_blocks is not None:
@@ -74,5 +80,5 @@ def fused_linear(value, packed, shape, kind, bias=None, *, q8_blocks=None, q8_ti
             w = q8_blocks.reshape(-1)
         else:
             w = L.q4_0_to_q8_0(w, n, k)
-    out = L.gemm(x, w, n, bias=b32, mode=L.MODE_DEQUANT, flags=flags)
+    out = L.gemm(x, w, n, bias=bias, mode=L.MODE_DEQUANT, flags=flags)
     return out.reshape(*value.shape[:-1], n)

@@ -145,6 +145,29 @@ def test_packed_linear_runs_its_tiled_copy_with_the_same_bits(kind):
     assert layer._q8_tiled is not first
 
 
+@pytest.mark.parametrize("kind", [T.Q8_0, T.Q4_0, T.Q4_K])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,n,k", [(1, 520, 512), (16, 130, 768), (17, 132, 256), (300, 520, 512), (3000, 1536, 256)])
+def test_packed_linear_widens_its_bias_in_the_kernel(kind, dtype, rows, n, k):
+    # the layer's bias in its own type, aligned, two bytes off (as a view) and strided: the bits of the fp32 bias
+    import idolq_lib as L
+    code = {T.Q8_0: 8, T.Q4_0: 4, T.Q4_K: 44}[kind]
+    gen = torch.Generator(device=DEV).manual_seed(rows)
+    size = n * k // 32 * 34 if code == 8 else n * k // 32 * 18 if code == 4 else n * k // 256 * 144
+    packed = torch.randint(0, 256, (size,), device=DEV, generator=gen, dtype=torch.int32).to(torch.uint8)
+    step = {8: 34, 4: 18, 44: 144}[code]
+    packed.view(-1, step)[:, 1] = 0x20  # finite scales (and Q4_K minimums)
+    if code == 44:
+        packed.view(-1, step)[:, 3] = 0x20
+    x = torch.randn(rows, k, device=DEV, dtype=dtype, generator=gen)
+    wide = torch.randn(2 * n + 1, device=DEV, dtype=dtype, generator=gen)
+    tiled = L.tile_q8_0(packed, n, k) if code == 8 else None
+    for bias in (wide[:n].clone(), wide[1:n + 1], wide[:2 * n:2]):
+        got = fused_linear(x, packed, (n, k), code, bias, q8_tiled=tiled)
+        plain = fused_linear(x, packed, (n, k), code, None, q8_tiled=tiled)
+        assert torch.equal(got, (plain.float() + bias.float()).to(dtype))
+
+
 def test_fp16_large_m_q8_0_adds_the_bias_before_its_rounding():
     # tools/idol_triton.py:112-117: fp16 activations, m >= 4096, n >= 1024, k >= 1024 go through F.linear, whose fused
     # bias enters the fp32 accumulator before the single rounding to fp16; below that size (and in bf16) the product
