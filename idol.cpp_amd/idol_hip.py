@@ -42,13 +42,13 @@ def fused_linear(value, packed, shape, kind, bias=None, *, q8_blocks=None, q8_ti
         raise ValueError('invalid packed linear dimensions')
     if bias is not None and (bias.shape != (n,) or bias.device != value.device or bias.dtype != value.dtype):
         raise ValueError('invalid fused linear bias')
-    x = value.reshape(-1, k)
+    x = value if value.dim() == 2 else value.reshape(-1, k)
     if x.shape[0] and x.stride(-1) != 1:
         x = x.contiguous()
     m = x.shape[0]
     if not m:
         return torch.empty((*value.shape[:-1], n), device=value.device, dtype=value.dtype)
-    w = packed.reshape(-1)
+    w = packed if packed.dim() == 1 else packed.reshape(-1)
     # The bias enters the epilogue as fp32, as the reference loads it (an exact widening): the small-m, tiled and Q4_K
     # kernels widen it themselves where its entries are whole vectors; the other row-major kernels take fp32.
     whole = bias is None or (bias.is_contiguous() and bias.data_ptr() % 16 == 0)
@@ -58,7 +58,7 @@ def fused_linear(value, packed, shape, kind, bias=None, *, q8_blocks=None, q8_ti
         if x.data_ptr() % 16:  # the Q4_K kernel reads 16-byte aligned rows (k % 256 == 0): only a view can miss it
             x = x.clone()
         out = L.q4_k_gemm(x, w, n, bias=bias, flags=L.FLAG_ROUND_BEFORE_BIAS)
-        return out.reshape(*value.shape[:-1], n)
+        return out if value.dim() == 2 else out.reshape(*value.shape[:-1], n)
     # the reference's F.linear branch adds the bias before its one rounding; everywhere else the product is rounded
     # first
     dense_branch = kind == KIND_Q8_0 and value.dtype == torch.float16 and m >= 4096 and n >= 1024 and k >= 1024
@@ -72,7 +72,7 @@ def fused_linear(value, packed, shape, kind, bias=None, *, q8_blocks=None, q8_ti
         if q8_tiled.numel() != L.tiled_q8_0_bytes(n, k) or q8_tiled.device != value.device:
             raise ValueError('invalid packed linear dimensions')
         out = L.gemm(x, q8_tiled.reshape(-1), n, bias=bias, mode=L.MODE_DEQUANT, flags=flags, tiled=True)
-        return out.reshape(*value.shape[:-1], n)
+        return out if value.dim() == 2 else out.reshape(*value.shape[:-1], n)
     if kind == KIND_Q4_0:
         if q8_blocks is not None:
             if q8_blocks.numel() != n * (k // 32) * 34 or q8_blocks.device != value.device:
@@ -81,4 +81,4 @@ def fused_linear(value, packed, shape, kind, bias=None, *, q8_blocks=None, q8_ti
         else:
             w = L.q4_0_to_q8_0(w, n, k)
     out = L.gemm(x, w, n, bias=bias, mode=L.MODE_DEQUANT, flags=flags)
-    return out.reshape(*value.shape[:-1], n)
+    return out if value.dim() == 2 else out.reshape(*value.shape[:-1], n)

@@ -103,12 +103,20 @@ def _check(rc):
         raise IdolqError(msg)
 
 
+# What every call pays on the host is kept short: small products take less time on the device than a call takes here.
+# Pointers and streams go to ctypes as plain integers (their argument types are c_void_p), the stream's handle comes
+# without a Stream object around it, and a tensor's device is compared by its index.
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _stream(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    if _raw_stream is None or device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
 
 
 def _code(t):
@@ -120,9 +128,12 @@ def _code(t):
 
 def _row_stride(t):
     """Row stride (elements) of a 2-D tensor whose last dimension is unit-stride."""
-    if t.dim() != 2 or (t.shape[1] > 1 and t.stride(1) != 1):
+    if t.dim() != 2:
         raise ValueError("expected a 2-D tensor with a unit-stride last dimension")
-    return max(t.stride(0), t.shape[1]) if t.shape[0] > 1 else t.shape[1]
+    (rows, cols), (row, col) = t.shape, t.stride()
+    if cols > 1 and col != 1:
+        raise ValueError("expected a 2-D tensor with a unit-stride last dimension")
+    return max(row, cols) if rows > 1 else cols
 
 
 def _require_shape(t, rows, cols, name):
@@ -130,30 +141,32 @@ def _require_shape(t, rows, cols, name):
     row stride, so a shorter or narrower view cannot send the kernel past the end of its memory."""
     if t is None:
         return
-    if t.dim() != 2 or tuple(t.shape) != (rows, cols):
+    if t.shape != (rows, cols):
         raise ValueError(f"{name} must be a [{rows}, {cols}] tensor, got {list(t.shape)}")
-    if cols > 1 and t.stride(1) != 1:
+    row, col = t.stride()
+    if cols > 1 and col != 1:
         raise ValueError(f"{name} needs a unit-stride last dimension")
-    if rows > 1 and t.stride(0) < cols:
-        raise ValueError(f"{name} rows overlap (row stride {t.stride(0)} < {cols})")
+    if rows > 1 and row < cols:
+        raise ValueError(f"{name} rows overlap (row stride {row} < {cols})")
 
 
 def _require_cuda(*tensors):
-    dev = None
+    first, index = None, -1
     for t in tensors:
         if t is None:
             continue
         if not t.is_cuda:
             raise ValueError("libidolq works on GPU tensors")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
+        if first is None:
+            first, index = t, t.get_device()
+        elif t.get_device() != index:
             raise ValueError("all tensors must be on the same device")
-    return dev
+    return None if first is None else first.device
 
 
 def q8_0_bytes(n, k):
-    return int(load().idolq_q8_0_bytes(n, k))
+    """Bytes of an [n, k] Q8_0 matrix (idolq_q8_0_bytes; 0 unless k is a multiple of 32)."""
+    return n * (k // Q8_0_BLOCK) * Q8_0_BYTES if n >= 0 and k >= 0 and k % Q8_0_BLOCK == 0 else 0
 
 
 _split_workspaces = {}
@@ -196,7 +209,7 @@ def gemm(x, w, n_total, n_offset=0, n=None, bias=None, residual=None, act=ACT_NO
     dev = _require_cuda(x, w, bias, residual, out, workspace)
     if w.dtype != torch.uint8:
         raise ValueError("Q8_0 weights are a uint8 tensor")
-    wbytes = int(lib.idolq_q8_0_tiled_bytes(n_total, k)) if tiled else q8_0_bytes(n_total, k)
+    wbytes = tiled_q8_0_bytes(n_total, k) if tiled else q8_0_bytes(n_total, k)
     if w.numel() != wbytes or not w.is_contiguous():
         raise ValueError("Q8_0 weight size does not match its shape")
     if tiled:
@@ -206,13 +219,14 @@ def gemm(x, w, n_total, n_offset=0, n=None, bias=None, residual=None, act=ACT_NO
     if bias is not None and (bias.dim() != 1 or bias.numel() != n_total or not bias.is_contiguous()):
         raise ValueError("bias must be a contiguous vector of n_total values")
     eff_mode = mode if mode != MODE_AUTO else (MODE_EXACT if x.dtype == torch.float32 else MODE_DEQUANT)
-    ws_bytes = int(lib.idolq_q8_0_gemm_workspace(m, k, eff_mode))
-    if eff_mode == MODE_EXACT and not tiled:
-        ws_bytes = 0   # the row-major EXACT kernel takes none
-    elif eff_mode in (MODE_INT8, MODE_EXACT) and not (tiled and split):
-        # the INT8 codes and scales or the EXACT high and low parts alone (the rest of the workspace is the tiled
-        # path's split room)
-        ws_bytes -= int(lib.idolq_q8_0_gemm_workspace(m, k, MODE_DEQUANT))
+    if eff_mode == MODE_EXACT and not tiled or eff_mode == MODE_DEQUANT and not split and workspace is None:
+        ws_bytes = 0   # the row-major EXACT kernel takes none, DEQUANT without one runs whole tiles
+    else:
+        ws_bytes = int(lib.idolq_q8_0_gemm_workspace(m, k, eff_mode))
+        if eff_mode in (MODE_INT8, MODE_EXACT) and not (tiled and split):
+            # the INT8 codes and scales or the EXACT high and low parts alone (the rest of the workspace is the tiled
+            # path's split room)
+            ws_bytes -= int(lib.idolq_q8_0_gemm_workspace(m, k, MODE_DEQUANT))
     if ws_bytes and (workspace is None or workspace.numel() * workspace.element_size() < ws_bytes):
         if eff_mode == MODE_DEQUANT:
             workspace = _split_workspace(x.device, ws_bytes) if split else None
@@ -242,7 +256,7 @@ def q4_k_gemm(x, w, n_total, n_offset=0, n=None, bias=None, residual=None, act=A
     _require_shape(out, m, n, "out")
     _require_shape(residual, m, n, "residual")
     dev = _require_cuda(x, w, bias, residual, out)
-    if w.dtype != torch.uint8 or w.numel() != int(lib.idolq_q4_k_bytes(n_total, k)) or not w.is_contiguous():
+    if w.dtype != torch.uint8 or w.numel() != q4_k_bytes(n_total, k) or not w.is_contiguous():
         raise ValueError("Q4_K weight size does not match its shape")
     if bias is not None and (bias.dim() != 1 or bias.numel() != n_total or not bias.is_contiguous()):
         raise ValueError("bias must be a contiguous vector of n_total values")
@@ -260,9 +274,14 @@ def q4_k_gemm(x, w, n_total, n_offset=0, n=None, bias=None, residual=None, act=A
     return out
 
 
+def q4_k_bytes(n, k):
+    """Bytes of an [n, k] Q4_K matrix (idolq_q4_k_bytes; 0 unless k is a multiple of 256)."""
+    return n * (k // 256) * 144 if n >= 0 and k > 0 and k % 256 == 0 else 0
+
+
 def tiled_q8_0_bytes(n, k):
     """Bytes of the tiled layout of an [n, k] Q8_0 matrix (rows padded to a multiple of 32; 0 unless k % 64 == 0)."""
-    return int(load().idolq_q8_0_tiled_bytes(n, k))
+    return (n + 31) // 32 * (k // 64) * 2176 if n >= 0 and k > 0 and k % 64 == 0 else 0
 
 
 def tile_q8_0(w, n, k):

@@ -511,6 +511,6 @@ def test_attention_fp32_without_a_workspace_takes_the_kernel_that_cuts_keys_insi
     assert lib.idolq_attention_f32_workspace(1, lq, lk, heads, 48) == 0
     out = torch.empty((lq, dim), device=DEV)
     assert lib.idolq_attention(L._ptr(qd), L._ptr(kd), L._ptr(vd), L.F32, 1, lq, lk, heads, hd, dim, dim, 0, 0,
-                               L._ptr(out), L.F32, dim, 0, L._stream(DEV)) == 0
+                               L._ptr(out), L.F32, dim, 0, L._stream(out.device)) == 0
     torch.cuda.synchronize()
     assert norm_rel(out.cpu().numpy(), _attention64(q, k, v, heads, hd)) < 2e-6
