@@ -59,6 +59,41 @@ __global__ __launch_bounds__(256) void q8_dequant_kernel(const uint8_t* __restri
     }
 }
 
+// The same values for 16-byte aligned blocks (the output always is): a workgroup takes 256 blocks, brings their 8704 bytes into LDS
+// as 16-byte pieces and writes them out 8 values a thread, both in whole lines (a thread per block reads 34 single
+// bytes and writes 64-byte strides). Bound by HBM: 6144 x 1536 to bf16, 29 MB, 11.7 -> 8.3 us under the tracer.
+constexpr int kDequantBlocks = 256;
+
+template <typename T>
+__global__ __launch_bounds__(256) void q8_dequant_lines_kernel(const uint8_t* __restrict__ w, int64_t blocks,
+                                                               T* __restrict__ out) {
+    constexpr int kBytes = kDequantBlocks * kQ8Bytes;
+    __shared__ __attribute__((aligned(16))) uint16_t lds[kBytes / 2];
+    const int64_t b0 = (int64_t)blockIdx.x * kDequantBlocks;
+    const int count = (int)(blocks - b0 < kDequantBlocks ? blocks - b0 : kDequantBlocks), bytes = count * kQ8Bytes;
+    const uint8_t* src = w + b0 * kQ8Bytes;
+    for (int i = threadIdx.x; i < bytes / 16; i += 256)
+        reinterpret_cast<uint4*>(lds)[i] = reinterpret_cast<const uint4*>(src)[i];
+    for (int i = bytes / 16 * 8 + threadIdx.x; i < bytes / 2; i += 256) lds[i] = reinterpret_cast<const uint16_t*>(src)[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int u = threadIdx.x + 256 * i, b = u >> 2, c = u & 3;
+        if (b >= count) break;
+        const uint16_t* blk = lds + b * (kQ8Bytes / 2);
+        const float d = half_bits_to_float(blk[0]);
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint16_t two = blk[1 + 4 * c + e];
+            v[2 * e] = (float)(int8_t)(two & 0xff) * d;
+            v[2 * e + 1] = (float)(int8_t)(two >> 8) * d;
+        }
+        store8<std::is_same<T, float>::value ? IDOLQ_F32 : std::is_same<T, __bf16>::value ? IDOLQ_BF16 : IDOLQ_F16>(
+            out, (b0 + b) * kQ8Block + 8 * c, v);
+    }
+}
+
 // ------------------------------------------------------------------------------------------------ Q8_0 quantizer
 // One thread per 32-value block of an fp32 [n x k] matrix: d = amax / 127, id = d ? 1 / d : 0,
 // q = round-half-away-from-zero(x * id), d stored as fp16 (ggml's quantize_row_q8_0_ref, the rule gguf-py's
@@ -369,6 +404,17 @@ extern "C" int idolq_q8_0_dequant(const uint8_t* w, int64_t n, int64_t k, void* 
     if (blocks == 0) return IDOLQ_OK;
     if (!w || !out) return fail(IDOLQ_EINVAL, "w and out must be non-null");
     if (reinterpret_cast<uintptr_t>(out) % 16 != 0) return fail(IDOLQ_EINVAL, "out must be 16-byte aligned");
+    if (reinterpret_cast<uintptr_t>(w) % 16 == 0) {
+        const dim3 grid((unsigned)((blocks + kDequantBlocks - 1) / kDequantBlocks));
+        hipStream_t s = static_cast<hipStream_t>(stream);
+        if (out_dtype == IDOLQ_F32)
+            hipLaunchKernelGGL(q8_dequant_lines_kernel<float>, grid, dim3(256), 0, s, w, blocks, static_cast<float*>(out));
+        else if (out_dtype == IDOLQ_BF16)
+            hipLaunchKernelGGL(q8_dequant_lines_kernel<__bf16>, grid, dim3(256), 0, s, w, blocks, static_cast<__bf16*>(out));
+        else
+            hipLaunchKernelGGL(q8_dequant_lines_kernel<_Float16>, grid, dim3(256), 0, s, w, blocks, static_cast<_Float16*>(out));
+        return check_launch("q8_dequant_lines_kernel");
+    }
     hipLaunchKernelGGL(q8_dequant_kernel, dim3((unsigned)((blocks + 255) / 256)), dim3(256), 0,
                        static_cast<hipStream_t>(stream), w, blocks, out, out_dtype);
     return check_launch("q8_dequant_kernel");

@@ -95,6 +95,23 @@ def test_int8_mfma_block_dots_are_bit_exact(m, n, k, off, cnt):
     assert np.array_equal(got, O.block_dots(qa, w, k, off, cnt))
 
 
+@pytest.mark.parametrize("n,k", [(1, 32), (3, 160), (255, 32), (257, 32), (64, 4096)])
+def test_dequant_writes_every_block(n, k):
+    # whole and partial groups of 256 blocks, all codes and a denormal scale among them, aligned and (two bytes off)
+    # not, each output type: the bits of the product rounded once
+    rng = np.random.default_rng(n + k)
+    w = rng.integers(0, 256, (n * k // 32, 34)).astype(np.uint8)
+    w[:, 1] &= 0x3b  # finite scales
+    w[0, :2] = (1, 0)
+    buf = torch.zeros(w.size + 2, dtype=torch.uint8, device=DEV)
+    buf[2:] = to_dev(w.reshape(-1))
+    d = np.ascontiguousarray(w[:, :2]).view(np.float16).astype(np.float32)
+    want = torch.from_numpy((w[:, 2:].view(np.int8) * d).reshape(n, k))
+    for dt in (torch.float32, torch.bfloat16, torch.float16):
+        for blocks in (to_dev(w.reshape(-1)), buf[2:]):
+            assert torch.equal(L.dequant(blocks, n, k, dt).cpu(), want.to(dt)), dt
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 33, 32), (16, 64, 160), (17, 63, 128), (65, 129, 224), (130, 64, 4096),
                                    (2049, 2050, 96), (1, 4096, 256)])
 @pytest.mark.parametrize("skew", [0, 2])
