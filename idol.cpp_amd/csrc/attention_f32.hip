@@ -4,9 +4,9 @@
 // fp32 product made of three fp16 products has 5 times the rate. x = h + l with h = fp16(x) and l = fp16(x - h), both
 // rounded to nearest (x - h is exact in fp32), holds 22 to 24 bits of x; a product keeps hh, hl and lh and drops ll,
 // at most 2^-22 of it. Everything is accumulated in fp32, a rounding per 16 products where the fp32 instruction
-// rounds after 2, so the result is closer to fp64 than that kernel's over the sizes that were measured (64 to 8192
-// keys). Powers of two keep the operands
-// in fp16's range: one per query of Q, per key place of K, per column of V, and 2^4 for the probabilities (more would
+// rounds after 2, so the result's 2-norm error is below that kernel's over the sizes that were measured (64 to 8192
+// keys; the largest single error too, but for 2048 x 8192 x 16 heads of 32: 9.2e-6 of the rms, there 8.8e-6).
+// Powers of two keep the operands in fp16's range: one per query of Q, per key place of K, per column of V, and 2^4 for the probabilities (more would
 // cost the exponent's argument bits). So a value of Q, K or V loses bits of its low part only below 2^-12 of the
 // largest of its row or column, a probability below 2^-7 of its query's largest, and what is lost is below 2^-34 and
 // 2^-29 of that largest.
@@ -547,8 +547,9 @@ __global__ __launch_bounds__(256) void attn_f32_combine(AttnParams p, int parts,
 // The cheapest of the kernel's forms (waves per workgroup), numbers of parts and, with waves 0, attn_f32_mfma, from
 // measured times in microseconds at head_dim 64: a tile step of a workgroup alone on its CU, of two (4 waves) and of
 // the 8-wave form, one and a half steps to start, and the merge (a launch and the partials written and read back);
-// attn_f32_mfma steps 32 keys in each of its 4 waves in 2.85, without the split's start. 300 queries, 16 heads, 64 /
-// 231 / 700 keys (this kernel against that one): 9.8 / 16.4 / 17.6 against 8.2 / 12.7 / 30 us.
+// attn_f32_mfma steps 32 keys in each of its 4 waves in 2.85, without the split's start. At 16 heads of 64 this
+// kernel against that one: 300 queries x 64 keys 9.8 against 8.2 us, 328 x 231 16.4 against 12.7, 128 x 700 17.0
+// against 22.8.
 AttnF32Plan attn_f32_plan(int64_t batch, int64_t lq, int64_t lk, int64_t heads, int64_t head_dim) {
     const int64_t cus = cu_count(), tiles = (lk + kTile - 1) / kTile;
     const double depth = head_dim == 64 ? 1.0 : 0.75;
