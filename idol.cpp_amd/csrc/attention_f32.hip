@@ -297,12 +297,11 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
         for (int c4 = 0; c4 < DC; ++c4) s = mfma(kf[1][c4], qf[0][c4], s);
 #pragma unroll
         for (int c4 = 0; c4 < DC; ++c4) s = mfma(kf[0][c4], qf[0][c4], s);
-        if (MASK) {
-            const int valid = (int)(lk - k0);
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                if (8 * (r >> 2) + 4 * half + (r & 3) >= valid) s[r] = -INFINITY;
-        }
+        // keys past lk have no score: decided on the scaled scores, since a unit (ck) of tiny operands may be 0
+        const int valid = MASK ? (int)(lk - k0) : kTile;
+        auto scored = [&](int r, float x) __attribute__((always_inline)) {
+            return MASK && 8 * (r >> 2) + 4 * half + (r & 3) >= valid ? -INFINITY : x;
+        };
         // The maximum mc (kept less kOffset) is the first tile's, raised only where a lane's probabilities of a tile
         // sum to 2^kSumBits or more, infinity and NaN included: no maximum is taken of the other tiles, the sum is
         // needed anyway, and every probability stays inside fp16 (a wave-uniform branch). While every score was -inf,
@@ -310,12 +309,12 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
         if (FIRST) {
             float mx = -INFINITY;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r] * ck[r]);
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, scored(r, s[r] * ck[r]));
             mc = fmaxf(mx, __shfl_xor(mx, 32)) - kOffset;
         }
         const float sub = mc == -INFINITY ? 0.0f : mc;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = fmaf(s[r], ck[r], -sub);
+        for (int r = 0; r < 16; ++r) s[r] = scored(r, fmaf(s[r], ck[r], -sub));
         f32x16 pr;
         float lt;
         auto probabilities = [&]() __attribute__((always_inline)) {

@@ -514,3 +514,31 @@ def test_attention_fp32_without_a_workspace_takes_the_kernel_that_cuts_keys_insi
                                L._ptr(out), L.F32, dim, 0, L._stream(out.device)) == 0
     torch.cuda.synchronize()
     assert norm_rel(out.cpu().numpy(), _attention64(q, k, v, heads, hd)) < 2e-6
+
+
+# lq, heads, lk: a cut key range, and one whose query tiles fill the device
+F32_RANGES = [(200, 2, 1507), (4096, 16, 421)]
+
+
+def _attention_f32_inputs(seed, lq, lk, dim):
+    rng = np.random.default_rng(seed)
+    return [rng.normal(0, 1, (n, dim)).astype(np.float32) for n in (lq, lk, lk)]
+
+
+def _attention_f32_head(q, k, v, heads, hd):
+    """fp32 attention of [n, heads * hd] arrays: head 0 of 96 queries, and the same in fp64."""
+    lq, lk, dim = len(q), len(k), heads * hd
+    out = torch.empty((lq, dim), device=DEV)
+    L.attention(to_dev(q), to_dev(k), to_dev(v), 1, lq, lk, heads, hd, dim, dim, 0, 0, out, dim, 0)
+    rows = np.linspace(0, lq - 1, 96).astype(int)
+    return out.cpu().numpy()[rows, :hd], _attention64(q[rows, :hd], k[:, :hd], v[:, :hd], 1, hd)
+
+
+@pytest.mark.parametrize("hd", [32, 64])
+@pytest.mark.parametrize("lq,heads,lk", F32_RANGES)
+def test_attention_fp32_of_vanishing_scores_masks_the_keys_past_the_end(hd, lq, heads, lk):
+    # Q and K of 1e-20: every score is 0, as are the units of the scaled operands, and the result is the mean of V over
+    # the lk keys there are
+    q, k, v = _attention_f32_inputs(hd + lk, lq, lk, heads * hd)
+    got, want = _attention_f32_head(q * np.float32(1e-20), k * np.float32(1e-20), v, heads, hd)
+    assert norm_rel(got, want) < 2e-6
