@@ -43,19 +43,22 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 2 : 1) void q8_gemm_i8_ker
 
     // The places of this thread's units, which no stage changes: byte offsets into x's codes, the weight window and the
     // scales, to which a stage adds a scalar offset (a full stage's loads and stores are then free of vector
-    // arithmetic), and offsets into LDS. Rows outside x or the window, whose results are not written, read row 0.
-    uint32_t a_off[kAPer], w_off[kWPer], s_off[kSPer];
+    // arithmetic), and offsets into LDS. Rows outside x or the window, whose results are not written, read row 0. The
+    // GEMM's entry point keeps codes and window below 2^32 bytes; the block sums' does not, and DOTS reads by pointer.
+    typedef typename std::conditional<DOTS, int64_t, uint32_t>::type Offset;
+    Offset a_off[kAPer], w_off[kWPer];
+    uint32_t s_off[kSPer];
     int a_at[kAPer], w_at[kWPer], s_at[kSPer];
 #pragma unroll
     for (int i = 0; i < kAPer; ++i) {
         const int u = tid + i * THREADS, row = u / (kStageK / 16), cu = u % (kStageK / 16);
-        a_off[i] = (m0 + row < p.m ? (uint32_t)(m0 + row) * (uint32_t)p.k : 0) + cu * 16;
+        a_off[i] = (m0 + row < p.m ? (Offset)(m0 + row) * p.k : 0) + cu * 16;
         a_at[i] = row * kAPitch + cu * 16;
     }
 #pragma unroll
     for (int i = 0; i < kWPer; ++i) {
         const int u = tid + i * THREADS, row = u / kUnitsPerRow, part = u % kUnitsPerRow;
-        w_off[i] = (row < BN && n0 + row < p.n ? (uint32_t)((int64_t)(n0 + row) * p.row_bytes) : 0) + part * (W4 ? 4 : 2);
+        w_off[i] = (row < BN && n0 + row < p.n ? (Offset)((int64_t)(n0 + row) * p.row_bytes) : 0) + part * (W4 ? 4 : 2);
         w_at[i] = row * kWPitch * (W4 ? 1 : 2) + part;
     }
 #pragma unroll
@@ -82,8 +85,11 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 2 : 1) void q8_gemm_i8_ker
 #pragma unroll
         for (int i = 0; i < kAPer; ++i) {
             const bool ok = in((tid + i * THREADS) % (kStageK / 16) / 2);
-            r.a[i] = __builtin_bit_cast(
-                uint4, __builtin_amdgcn_raw_buffer_load_b128(ra, ok ? a_off[i] : 0, ok ? blk0 * kQ8Block : 0, 0));
+            if constexpr (DOTS)
+                r.a[i] = *reinterpret_cast<const uint4*>(p.qa + (ok ? a_off[i] + blk0 * kQ8Block : 0));
+            else
+                r.a[i] = __builtin_bit_cast(
+                    uint4, __builtin_amdgcn_raw_buffer_load_b128(ra, ok ? a_off[i] : 0, ok ? blk0 * kQ8Block : 0, 0));
             if (TAIL && !ok) r.a[i] = make_uint4(0, 0, 0, 0);
         }
 #pragma unroll
@@ -91,8 +97,13 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 2 : 1) void q8_gemm_i8_ker
             // (a dword straddles the first two or the last two blocks of a stage; W4 rows hold an even number)
             const bool ok = in((tid + i * THREADS) % kUnitsPerRow * (W4 ? 4 : 2) / kQ8Bytes);
             const int at = ok ? (int)w_off[i] : 0, st_off = ok ? blk0 * kQ8Bytes : 0;
-            r.w[i] = W4 ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rw, at, st_off, 0)
-                        : (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rw, at, st_off, 0);
+            if constexpr (DOTS) {
+                const uint8_t* src = p.w + (ok ? w_off[i] + st_off : 0);
+                r.w[i] = W4 ? *reinterpret_cast<const uint32_t*>(src) : *reinterpret_cast<const uint16_t*>(src);
+            } else {
+                r.w[i] = W4 ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rw, at, st_off, 0)
+                            : (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rw, at, st_off, 0);
+            }
             if (TAIL && !ok) r.w[i] = 0;
         }
         if (!DOTS)

@@ -614,3 +614,21 @@ def test_int8_on_tiled_weights_with_strided_activation_rows():
     til = L.gemm(x, wt, n, bias=bt, mode=L.MODE_INT8, out_dtype=torch.float32, tiled=True)
     torch.cuda.synchronize()
     assert torch.equal(raw, til)
+
+
+def test_block_dots_past_two_to_the_32_bytes_of_codes():
+    # codes of 2^32 bytes and more: the rows past them are read at 64-bit offsets
+    lib = L.load()
+    m, k, n = 65600, 65536, 3
+    rng = np.random.default_rng(32)
+    tail = rng.integers(-127, 128, (64, k), dtype=np.int8)
+    qa = torch.zeros((m, k), device=DEV, dtype=torch.int8)
+    qa[m - 64:] = torch.from_numpy(tail).to(DEV)
+    w = O.q8_0_quantize(rng.normal(0, 1, (n, k)).astype(np.float32))
+    wd = torch.from_numpy(w).to(DEV)
+    dots = torch.full((m, n, k // 32), -1, device=DEV, dtype=torch.int32)
+    assert lib.idolq_q8_0_block_dots(L._ptr(qa), m, k, L._ptr(wd), n, 0, n, L._ptr(dots), L._stream(dots.device)) == 0
+    codes = w.reshape(n, k // 32, 34)[:, :, 2:].view(np.int8).astype(np.int32)
+    want = np.einsum("mbe,nbe->mnb", tail.reshape(64, k // 32, 32).astype(np.int32), codes)
+    assert np.array_equal(dots[m - 64:].cpu().numpy(), want)
+    assert not dots[:m - 64].any()
