@@ -1,32 +1,31 @@
-// fp32 attention on the fp16 matrix cores: every fp32 operand as the sum of two fp16 values.
+// fp32 attention on the 16-bit matrix cores: fp32 operands as sums of 16-bit values.
 //
-// The fp32 matrix instructions (v_mfma_f32_32x32x2_f32) take 64 cycles for the products the fp16 ones do in 4, so an
-// fp32 product made of three fp16 products has 5 times the rate. x = h + l with h = fp16(x) and l = fp16(x - h), both
-// rounded to nearest (x - h is exact in fp32), holds 22 to 24 bits of x; a product keeps hh, hl and lh and drops ll,
-// at most 2^-22 of it. Everything is accumulated in fp32, a rounding per 16 products where the fp32 instruction
-// rounds after 2, so the result's 2-norm error is below that kernel's over the sizes that were measured (64 to 8192
-// keys; the largest single error too, but for 2048 x 8192 x 16 heads of 32: 9.2e-6 of the rms, there 8.8e-6).
-// Powers of two keep the operands in fp16's range: one per query of Q, per key place of K, per column of V, and 2^4 for the probabilities (more would
-// cost the exponent's argument bits). So a value of Q, K or V loses bits of its low part only below 2^-12 of the
-// largest of its row or column, a probability below 2^-7 of its query's largest, and what is lost is below 2^-34 and
-// 2^-29 of that largest.
+// The fp32 matrix instructions (v_mfma_f32_32x32x2_f32) take 64 cycles for the products the 16-bit ones do in 4.
 //
-// attn_f32_split<HD, NW>: a workgroup of NW waves owns 32 NW queries of one (batch, head) and a range of 32-key tiles. The tile's K and V are split once per workgroup on their way into LDS (K planes [key][d],
-// V planes transposed [d][key], the keys of a 16-chunk in the order in which a lane of the score accumulator holds
-// them), two tile buffers, one barrier per tile. Scores are computed transposed, S^T = K Q^T, so a lane holds 16
-// scores of one query and its probabilities, split in registers, are the B operand of O^T = V^T P^T.
+// The product with V holds both operands in three bf16 values h = bf16(x), m = bf16(x - h), l = bf16(x - h - m): all 24
+// bits of an fp32 value at its own exponent, so no value loses bits to a larger one beside it (a column of V may hold
+// 1e30 at a key of no weight, a query's weights may fall to 1e-30). Of the nine products lm, ml and ll are dropped, at
+// most 2^-25 of one; hh has an accumulator of its own, rounded once per 16 keys where the fp32 instruction rounds after
+// 2, and the five small ones share another.
 //
-// Scales: a tile is staged with the scales of the one before it, and each wave votes whether they still fit (largest
+// The scores hold Q and K as two fp16 values, h = fp16(x) and l = fp16(x - h), 22 to 24 bits of x, and drop ll, at most
+// 2^-22 of a product. Powers of two keep them in fp16's range, one per query of Q and one per key place of K.
+//
+// attn_f32_split<HD, NW>: a workgroup of NW waves owns 32 NW queries of one (batch, head) and a range of 32-key tiles.
+// The tile's K and V are split once per workgroup on their way into LDS (K planes [key][d], V planes transposed [d][key],
+// the keys of a 16-chunk in the order in which a lane of the score accumulator holds them), two tile buffers, one barrier
+// per tile. Scores are computed transposed, S^T = K Q^T, so a lane holds 16 scores of one query and its probabilities,
+// split in registers, are the B operand of O^T = V^T P^T.
+//
+// K's scales: a tile is staged with the scales of the one before it, and each wave votes whether they still fit (largest
 // magnitude of its values between 2^9 and 65000 after scaling). Where they do not, the workgroup takes new ones and
-// stages the tile again after the barrier (rare path, uniform over the workgroup); o moves to V's new scales exactly.
-// Infinite inputs, and K or Q of 2^60 and more, have no split: a workgroup that meets one starts its part again with
-// the fp32 matrix instructions on the inputs themselves (plain_part), so that infinities go through the arithmetic of
-// the plain fp32 product. A NaN splits into two and needs no path of its own.
+// stages the tile again after the barrier (rare path, uniform over the workgroup).
+// V of 2^70 and more and infinities, and K or Q of 2^60 and more, have no split: a workgroup that meets one starts its
+// part again with the fp32 matrix instructions on the inputs themselves (plain_part), so that infinities go through the
+// arithmetic of the plain fp32 product. A NaN splits into two or three and needs no path of its own.
 //
-// 1000 queries x 8192 keys x 16 heads of 64: 124 us (270 TFLOP/s), attn_f32_mfma 367 (92); 2-norm error against fp64
-// 5.6e-7, there 8.7e-7. The MFMAs of a tile and wave take 768 cycles and its vector instructions about 800 (counters:
-// hardly any of the two overlap), so what is left is mostly their sum: with 4 waves, whose staging is shared by half as
-// many queries, the same call takes 139 us, with a maximum per tile and one scale per tile 15% more.
+// 1000 queries x 8192 keys x 16 heads of 64, against attn_f32_mfma on the same box: 176 us, 424; 2-norm error against
+// fp64 3.6e-7, 8.6e-7; largest error 4.9e-6 of the rms, 8.2e-6.
 //
 // The key range is cut into parts (attn_f32_plan) where the query tiles alone leave CUs idle: each part writes its
 // maxima, sums and unnormalized output, and attn_f32_combine merges them.
@@ -42,13 +41,16 @@ constexpr int kVP = kTile + 8;  // elements per d row of a V plane (80 bytes: co
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 constexpr float kSplitLimit = 1152921504606846976.0f;  // 2^60
 constexpr float kScaledMin = 512.0f, kScaledMax = 65000.0f;
-// The probabilities are 2^(score + kOffset - maximum); a lane's 16 of a tile sum to less than 2^kSumBits, and to no more
-// than 2^(4 + kOffset) once the maximum is the largest.
-constexpr float kOffset = 4.0f;
-constexpr int kSumBits = 9;
+// A lane's 16 probabilities 2^(score - maximum) of a tile sum to less than 2^kSumBits (to at most 16 where the maximum
+// is the largest).
+constexpr int kSumBits = 5;
+// V is held times 2^24, so the lowest part of every normal value is one too; from 2^70 on it is not split (o stays
+// below 2^94 times the number of keys and 2^kSumBits).
+constexpr float kVScale = 16777216.0f, kVUnit = 1.0f / kVScale, kVLimit = 1180591620717411303424.0f;
 
 // Two values as fp16 pairs h, l.
 __device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& l) {
@@ -56,6 +58,19 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& 
     const float ra = fmaf((float)hv.x, -1.0f, a), rb = fmaf((float)hv.y, -1.0f, b);
     h = __builtin_bit_cast(uint32_t, hv);
     l = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{ra, rb}), f16x2));
+}
+
+// Two values as bf16 triples h, m, l: 8 bits each, all 24 bits of an fp32 value between them (down to 2^-109).
+__device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+    auto pack = [](float x, float y) __attribute__((always_inline)) {
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x, y}), bf16x2));
+    };
+    auto low = [](uint32_t w) __attribute__((always_inline)) { return __builtin_bit_cast(float, w << 16); };
+    auto high = [](uint32_t w) __attribute__((always_inline)) { return __builtin_bit_cast(float, w & 0xffff0000u); };
+    h = pack(a, b);
+    const float ra = a - low(h), rb = b - high(h);
+    m = pack(ra, rb);
+    l = pack(ra - low(m), rb - high(m));
 }
 
 // 2^e as fp32, e within [-126, 127]
@@ -71,6 +86,9 @@ __device__ __forceinline__ int scale_exp(float mx) {
 __device__ __forceinline__ f32x16 mfma(f16x8 a, f16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
+__device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
 
 // part_o [parts][batch][heads][lq][HD] unnormalized outputs, part_ml [...][lq][2] their maxima (base-2 domain) and sums
 template <int HD, int NW>
@@ -84,12 +102,9 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
     constexpr int EV = kTile * HD / (64 * NW);  // staged values per thread of K and of V
     constexpr int KP = HD + 8;    // elements per key row of a K plane (conflict-free 16-byte reads)
     __shared__ __attribute__((aligned(16))) uint16_t k_lds[2][2][kTile * KP];
-    __shared__ __attribute__((aligned(16))) uint16_t v_lds[2][2][HD * kVP];
+    __shared__ __attribute__((aligned(16))) uint16_t v_lds[2][3][HD * kVP];
     __shared__ uint32_t vote[2][NW];
-    __shared__ uint32_t col_max[2][HD];  // V's and o's largest finite magnitudes per column (their bits)
-    __shared__ int col_move[HD];         // the exponent by which o's column moves
-    __shared__ float col_unit[HD];       // what o's column is in units of
-    __shared__ float key_unit[kTile];    // the same of the scores of a key place
+    __shared__ float key_unit[kTile];  // what the scores of a key place are in units of
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, half = lane >> 5;
@@ -143,13 +158,13 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
     const int64_t tiles = (lk + kTile - 1) / kTile;
     const int64_t t0 = part * per, t1 = t0 + per < tiles ? t0 + per : tiles;
     float mc = -INFINITY, l_part = 0.0f;  // the running maximum (base-2 domain) and this lane's half of the sum
-    int ke = 0, ve = 0;  // the exponents of the scales of the thread's key of K and column of V
+    int ke = 0;  // the exponent of the scale of the thread's key of K
     float ck[16];
-    f32x16 o[DB];
+    f32x16 o[DB], small[DB];  // the sums of the products hh, and of the others
 #pragma unroll
     for (int t = 0; t < DB; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o[t][r] = 0.0f;
+        for (int r = 0; r < 16; ++r) o[t][r] = 0.0f, small[t][r] = 0.0f;
 
     // Staging. K: thread t takes EV values of a key, a row to HD / EV consecutive threads. V: thread t takes d row t % HD
     // and EV keys whose places in that row of the plane are contiguous: place 16 kc + 8 half + e holds key 16 kc +
@@ -195,12 +210,12 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
             }
         }
     };
-    // votes: 1 K beyond its scale's range, 2 some K within it, 4 some K not 0; 8, 16, 32 the same of V;
-    // 64 a value without a split (K of 2^60 or more, an infinite V; big: one of the wave's queries)
+    // votes: 1 K beyond its scale's range, 2 some K within it, 4 some K not 0; 64 a value without a split (K of 2^60
+    // or more, V of kVLimit or more; big: one of the wave's queries)
     auto stage_tile = [&](int buf, bool big) __attribute__((always_inline)) {
-        const float ks = pow2(ke), vs = pow2(ve);
+        const float ks = pow2(ke);
         float kmax = 0.0f, vmax = 0.0f;
-        uint32_t w[2][EV / 2];
+        uint32_t w[3][EV / 2];
         auto store = [&](uint16_t* dst, int pl) __attribute__((always_inline)) {
             if constexpr (EV == 8)
                 *reinterpret_cast<uint4*>(dst) = make_uint4(w[pl][0], w[pl][1], w[pl][2], w[pl][3]);
@@ -219,64 +234,34 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
         store(&k_lds[buf][1][skey * KP + sd], 1);
 #pragma unroll
         for (int e = 0; e < EV / 2; ++e) {
-            const float x = vr[2 * e] * vs, y = vr[2 * e + 1] * vs;
-            split2(x, y, w[0][e], w[1][e]);
-            vmax = fmaxf(vmax, fmaxf(fabsf(x), fabsf(y)));
+            split3(vr[2 * e] * kVScale, vr[2 * e + 1] * kVScale, w[0][e], w[1][e], w[2][e]);
+            vmax = fmaxf(vmax, fmaxf(fabsf(vr[2 * e]), fabsf(vr[2 * e + 1])));
         }
-        store(&v_lds[buf][0][vd * kVP + vplace], 0);
-        store(&v_lds[buf][1][vd * kVP + vplace], 1);
+#pragma unroll
+        for (int pl = 0; pl < 3; ++pl) store(&v_lds[buf][pl][vd * kVP + vplace], pl);
         auto any = [&](bool c) __attribute__((always_inline)) { return __builtin_amdgcn_ballot_w64(c) != 0; };
         uint32_t bits = any(kmax >= kScaledMin) ? 2u : 0u;  // every lane takes part
         bits |= any(kmax > kScaledMax) ? 1u : 0u;
         bits |= any(kmax > 0.0f) ? 4u : 0u;
-        bits |= any(vmax > kScaledMax) ? 8u : 0u;
-        bits |= any(vmax >= kScaledMin) ? 16u : 0u;
-        bits |= any(vmax > 0.0f) ? 32u : 0u;
-        bits |= any(big || kmax * pow2(-ke) >= kSplitLimit || vmax == INFINITY) ? 64u : 0u;
+        bits |= any(big || kmax * pow2(-ke) >= kSplitLimit || vmax >= kVLimit) ? 64u : 0u;
         if (lane == 0) vote[buf][wave] = bits;
     };
-    // New scales from the largest finite magnitudes of the tile in kr and vr, o moved to them, and the tile staged into
-    // buffer buf with them. Every wave takes part; col_max is 0 before and after.
+    // New scales from the largest finite magnitudes of the keys in kr, and the tile staged into buffer buf with them.
+    // Every wave takes part.
     auto rescale_tile = [&](int buf, bool big) __attribute__((always_inline)) {
         auto finite = [](float x) __attribute__((always_inline)) { return fabsf(x) < INFINITY ? fabsf(x) : 0.0f; };
-        auto bits = [](float x) __attribute__((always_inline)) { return __builtin_bit_cast(uint32_t, x); };
-        float km = 0.0f, vm = 0.0f;
+        float km = 0.0f;
 #pragma unroll
-        for (int i = 0; i < EV; ++i) {
-            km = fmaxf(km, finite(kr[i]));
-            vm = fmaxf(vm, finite(vr[i]));
-        }
+        for (int i = 0; i < EV; ++i) km = fmaxf(km, finite(kr[i]));
 #pragma unroll
         for (int off = 1; off < HD / EV; off <<= 1) km = fmaxf(km, __shfl_xor(km, off));
         ke = scale_exp(km);
         if (sd == 0) key_unit[skey] = pow2(-ke);
-        atomicMax(&col_max[0][vd], bits(vm));
-#pragma unroll
-        for (int t = 0; t < DB; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                atomicMax(&col_max[1][t * 32 + 8 * (r >> 2) + 4 * half + (r & 3)], bits(finite(o[t][r])));
-        __syncthreads();
-        // o stays below 2^101: against an o that large in its units, values the tile would need a finer scale for do
-        // not count
-        const int room = 100 + 127 - (int)(col_max[1][vd] >> 23);
-        int move = scale_exp(__builtin_bit_cast(float, col_max[0][vd])) - ve;
-        if (move > room) move = room;
-        ve += move;
-        if (tid < HD) col_move[vd] = move, col_unit[vd] = pow2(-ve);
-        __syncthreads();
-        if (tid < HD) col_max[0][vd] = 0, col_max[1][vd] = 0;
-#pragma unroll
-        for (int t = 0; t < DB; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = col_move[t * 32 + 8 * (r >> 2) + 4 * half + (r & 3)];  // up to 187: in two steps
-                o[t][r] = o[t][r] * pow2(m / 2) * pow2(m - m / 2);
-            }
+        __syncthreads();  // the units are in place, and every wave has read the votes that stage_tile writes again
 #pragma unroll
         for (int r = 0; r < 16; ++r) ck[r] = cq * key_unit[8 * (r >> 2) + 4 * half + (r & 3)];
         stage_tile(buf, big);
-        __syncthreads();  // the planes and votes are in place, col_max is clear
+        __syncthreads();  // the planes and votes are in place, the units have been read
     };
 
     // MASK: the last tile, with fewer than 32 keys; FIRST: the part's first tile, whose largest score sets the maximum
@@ -302,15 +287,14 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
         auto scored = [&](int r, float x) __attribute__((always_inline)) {
             return MASK && 8 * (r >> 2) + 4 * half + (r & 3) >= valid ? -INFINITY : x;
         };
-        // The maximum mc (kept less kOffset) is the first tile's, raised only where a lane's probabilities of a tile
-        // sum to 2^kSumBits or more, infinity and NaN included: no maximum is taken of the other tiles, the sum is
-        // needed anyway, and every probability stays inside fp16 (a wave-uniform branch). While every score was -inf,
-        // mc is -inf and 0 is subtracted: no weight.
+        // The maximum mc is the first tile's, raised only where a lane's probabilities of a tile sum to 2^kSumBits or
+        // more, infinity and NaN included: no maximum is taken of the other tiles, the sum is needed anyway (a
+        // wave-uniform branch). While every score was -inf, mc is -inf and 0 is subtracted: no weight.
         if (FIRST) {
             float mx = -INFINITY;
 #pragma unroll
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, scored(r, s[r] * ck[r]));
-            mc = fmaxf(mx, __shfl_xor(mx, 32)) - kOffset;
+            mc = fmaxf(mx, __shfl_xor(mx, 32));
         }
         const float sub = mc == -INFINITY ? 0.0f : mc;
 #pragma unroll
@@ -333,7 +317,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
             mx = fmaxf(mx, __shfl_xor(mx, 32));
             const bool none = mc == -INFINITY;
-            const float delta = none || mx > kOffset ? mx - kOffset : 0.0f;
+            const float delta = none || mx > 0.0f ? mx : 0.0f;
             if (delta > -INFINITY) {  // else still no score above -inf
                 const float alpha = none ? 0.0f : __builtin_amdgcn_exp2f(-delta);
                 mc = sub + delta;
@@ -341,7 +325,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
 #pragma unroll
                 for (int t = 0; t < DB; ++t)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
+                    for (int r = 0; r < 16; ++r) o[t][r] *= alpha, small[t][r] *= alpha;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) s[r] -= delta;
             }
@@ -350,23 +334,26 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
         l_part += lt;
 #pragma unroll
         for (int kc = 0; kc < 2; ++kc) {
-            uint32_t w[2][4];
+            uint32_t w[3][4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) split2(pr[8 * kc + 2 * e], pr[8 * kc + 2 * e + 1], w[0][e], w[1][e]);
-            f16x8 pf[2], vf[DB][2];
+            for (int e = 0; e < 4; ++e)
+                split3(pr[8 * kc + 2 * e], pr[8 * kc + 2 * e + 1], w[0][e], w[1][e], w[2][e]);
+            bf16x8 pf[3], vf[DB][3];
 #pragma unroll
-            for (int pl = 0; pl < 2; ++pl)
-                pf[pl] = __builtin_bit_cast(f16x8, make_uint4(w[pl][0], w[pl][1], w[pl][2], w[pl][3]));
+            for (int pl = 0; pl < 3; ++pl)
+                pf[pl] = __builtin_bit_cast(bf16x8, make_uint4(w[pl][0], w[pl][1], w[pl][2], w[pl][3]));
 #pragma unroll
             for (int t = 0; t < DB; ++t)
 #pragma unroll
-                for (int pl = 0; pl < 2; ++pl)
-                    vf[t][pl] = *reinterpret_cast<const f16x8*>(
+                for (int pl = 0; pl < 3; ++pl)
+                    vf[t][pl] = *reinterpret_cast<const bf16x8*>(
                         &v_lds[buf][pl][(t * 32 + col) * kVP + 16 * kc + 8 * half]);
+            // hl, lh, mm, hm, mh (lm, ml and ll, at most 2^-25 of a product, are dropped), and hh
+            constexpr int kSmall[5][2] = {{0, 2}, {2, 0}, {1, 1}, {0, 1}, {1, 0}};
 #pragma unroll
-            for (int t = 0; t < DB; ++t) o[t] = mfma(vf[t][0], pf[1], o[t]);
+            for (int i = 0; i < 5; ++i)
 #pragma unroll
-            for (int t = 0; t < DB; ++t) o[t] = mfma(vf[t][1], pf[0], o[t]);
+                for (int t = 0; t < DB; ++t) small[t] = mfma(vf[t][kSmall[i][0]], pf[kSmall[i][1]], small[t]);
 #pragma unroll
             for (int t = 0; t < DB; ++t) o[t] = mfma(vf[t][0], pf[0], o[t]);
         }
@@ -421,9 +408,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
         }
     };
 
-    if (tid < HD) col_max[0][tid] = 0, col_max[1][tid] = 0, col_unit[tid] = 1.0f;
     if (t0 < t1) load_tile(t0);
-    __syncthreads();
     if (t0 < t1) rescale_tile(0, qmax >= kSplitLimit);
     int buf = 0;
     bool plain = false;  // uniform over the workgroup
@@ -435,7 +420,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
         for (int w = 0; w < NW; ++w) votes |= vote[buf][w];
         votes = __builtin_amdgcn_readfirstlane(votes);
         if (votes & 64u) return false;
-        if ((votes & 9u) || (votes & 6u) == 4u || (votes & 48u) == 32u) rescale_tile(buf, false);
+        if ((votes & 1u) || (votes & 6u) == 4u) rescale_tile(buf, false);
         if (t + 1 < t1) load_tile(t + 1);
         if (active) compute(buf, t * kTile, mask_tag, first_tag);
         if (t + 1 < t1) stage_tile(buf ^ 1, false);
@@ -455,11 +440,13 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
     // the factor that takes a sum of weights to weights of at most 1, and the maximum those refer to
     float w = pow2(-kSumBits);
     mc += (float)kSumBits;
+#pragma unroll
+    for (int t = 0; t < DB; ++t) o[t] += small[t];
     if (plain) {
         w = 1.0f;
         if (active) plain_part();
     }
-    auto unit = [&](int d) __attribute__((always_inline)) { return plain ? 1.0f : col_unit[d]; };
+    const float unit = plain ? 1.0f : kVUnit;  // of o
 
     const float l = l_part + __shfl_xor(l_part, 32);
     if (qi >= lq) return;
@@ -472,7 +459,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
                 const int d = t * 32 + 2 * r + 4 * half;
                 f32x4 v;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = o[t][r + e] * w * unit(d + e);
+                for (int e = 0; e < 4; ++e) v[e] = o[t][r + e] * w * unit;
                 *reinterpret_cast<f32x4*>(part_o + row * HD + d) = v;
             }
         if (half == 0) *reinterpret_cast<f32x2*>(part_ml + 2 * row) = f32x2{mc, l * w};
@@ -487,7 +474,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
             const int d = t * 32 + 2 * r + 4 * half;
             float v[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = o[t][r + e] * inv * unit(d + e);
+            for (int e = 0; e < 4; ++e) v[e] = o[t][r + e] * inv * unit;
             if (p.out_vec) {
                 *reinterpret_cast<f32x4*>(static_cast<float*>(p.out) + obase + d) = f32x4{v[0], v[1], v[2], v[3]};
             } else {

@@ -542,3 +542,57 @@ def test_attention_fp32_of_vanishing_scores_masks_the_keys_past_the_end(hd, lq, 
     q, k, v = _attention_f32_inputs(hd + lk, lq, lk, heads * hd)
     got, want = _attention_f32_head(q * np.float32(1e-20), k * np.float32(1e-20), v, heads, hd)
     assert norm_rel(got, want) < 2e-6
+
+
+@pytest.mark.parametrize("hd", [32, 64])
+@pytest.mark.parametrize("lq,heads,lk", F32_RANGES)
+@pytest.mark.parametrize("tile", ["first", "middle", "last"])
+def test_attention_fp32_columns_of_v_beside_large_values_without_weight(hd, lq, heads, lk, tile):
+    # one key of weight e^-100 (or less) with a large V in some columns: each column keeps the accuracy that its own
+    # weighted values have in fp32 (see the tests above), since no operand is held relative to the largest of its column
+    q, k, v = _attention_f32_inputs(3 * hd + lk, lq, lk, heads * hd)
+    key = {"first": 7, "middle": lk // 2, "last": lk - 2}[tile]
+    q[:, 0] = 1.0
+    k[key] = 0.0
+    k[key, 0] = -800.0
+    for d, large in enumerate((1e4, 1e9, -1e12, 1e20, 1e30)):
+        v[key, d] = large
+    got, want = _attention_f32_head(q, k, v, heads, hd)
+    for d in range(hd):
+        assert norm_rel(got[:, d], want[:, d]) < 2e-6, d
+
+
+@pytest.mark.parametrize("hd", [32, 64])
+@pytest.mark.parametrize("lq,heads,lk", F32_RANGES)
+def test_attention_fp32_columns_of_v_that_start_at_zero_or_are_small(hd, lq, heads, lk):
+    # columns that are 0 or tiny in every other tile, small ones, and one that falls along the keys, beside columns of
+    # ordinary values
+    q, k, v = _attention_f32_inputs(5 * hd + lk, lq, lk, heads * hd)
+    even = (np.arange(lk) // 32) % 2 == 0
+    for d, scale in enumerate((1e-2, 1e-4, 1e-6, 1e-15)):
+        v[:, d] = np.where(even, 0.0, scale * v[:, d])
+        v[:, 4 + d] *= np.float32(scale * 1e-15)
+    v[even, 8] *= np.float32(2.0 ** -30)
+    v[:, 9] *= np.exp2(-np.arange(lk) / 8.0).astype(np.float32)
+    got, want = _attention_f32_head(q, k, v, heads, hd)
+    for d in range(hd):
+        assert norm_rel(got[:, d], want[:, d]) < 2e-6, d
+
+
+@pytest.mark.parametrize("hd", [32, 64])
+@pytest.mark.parametrize("peak", [3, 4000, 8189])
+def test_attention_fp32_small_weights_count_beside_a_dominant_key(hd, peak):
+    # one key 20.3 above 8190 equal ones (weights 1.5e-9 of its own): V is 0 for it and 1 for the others, 1 for all, and
+    # 1 with noise for the others; each column against fp64. A weight is off by what the exponent's argument, 29.3 in
+    # base 2, is: 2^-24 of it for the factor, the product and the difference each, 3.6e-6; the sum of the weights by up to
+    # 2^-25 a tile where the large one comes first, 3.8e-6 over a part of 128 tiles (these have fewer)
+    lq, lk, heads = 100, 8191, 2
+    q, k, v = _attention_f32_inputs(peak + hd, lq, lk, heads * hd)
+    q[:, :hd], k[:, :hd] = 0.0, 0.0
+    q[:, 0] = 1.0
+    k[peak, 0] = 20.3 * np.sqrt(hd)
+    v[:, 0], v[:, 1], v[:, 2] = 1.0, 1.0, 1.0 + v[:, 2]
+    v[peak, 0], v[peak, 2] = 0.0, 0.0
+    got, want = _attention_f32_head(q, k, v, heads, hd)
+    for d in range(hd):
+        assert norm_rel(got[:, d], want[:, d]) < 8e-6, d
