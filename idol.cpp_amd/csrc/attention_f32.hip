@@ -1,15 +1,12 @@
-// fp32 attention on the 16-bit matrix cores: fp32 operands as sums of 16-bit values.
+// fp32 attention on the bf16 matrix cores: every fp32 operand as the sum of three bf16 values.
 //
-// The fp32 matrix instructions (v_mfma_f32_32x32x2_f32) take 64 cycles for the products the 16-bit ones do in 4.
-//
-// The product with V holds both operands in three bf16 values h = bf16(x), m = bf16(x - h), l = bf16(x - h - m): all 24
-// bits of an fp32 value at its own exponent, so no value loses bits to a larger one beside it (a column of V may hold
-// 1e30 at a key of no weight, a query's weights may fall to 1e-30). Of the nine products lm, ml and ll are dropped, at
-// most 2^-25 of one; hh has an accumulator of its own, rounded once per 16 keys where the fp32 instruction rounds after
-// 2, and the five small ones share another.
-//
-// The scores hold Q and K as two fp16 values, h = fp16(x) and l = fp16(x - h), 22 to 24 bits of x, and drop ll, at most
-// 2^-22 of a product. Powers of two keep them in fp16's range, one per query of Q and one per key place of K.
+// The fp32 matrix instructions (v_mfma_f32_32x32x2_f32) take 64 cycles for the products the bf16 ones do in 4, so an
+// fp32 product made of six bf16 products has 2.7 times the rate. h = bf16(x), m = bf16(x - h) and l = bf16(x - h - m)
+// hold all 24 bits of x at its own exponent: no operand has a scale, and none loses bits to a larger one beside it (a
+// key may carry 1e12 in one channel, V 1e30 at a key of no weight, a query's weights may fall to 1e-30). Of the nine
+// products hh, hm, mh, mm, hl and lh are kept; lm, ml and ll are at most 2^-25 of one. Everything is accumulated in
+// fp32, hh of the product with V in an accumulator of its own: it rounds once per 16 keys where the fp32 instruction
+// rounds after 2, so the result's error is no larger than that kernel's (below).
 //
 // attn_f32_split<HD, NW>: a workgroup of NW waves owns 32 NW queries of one (batch, head) and a range of 32-key tiles.
 // The tile's K and V are split once per workgroup on their way into LDS (K planes [key][d], V planes transposed [d][key],
@@ -17,15 +14,16 @@
 // per tile. Scores are computed transposed, S^T = K Q^T, so a lane holds 16 scores of one query and its probabilities,
 // split in registers, are the B operand of O^T = V^T P^T.
 //
-// K's scales: a tile is staged with the scales of the one before it, and each wave votes whether they still fit (largest
-// magnitude of its values between 2^9 and 65000 after scaling). Where they do not, the workgroup takes new ones and
-// stages the tile again after the barrier (rare path, uniform over the workgroup).
-// V of 2^70 and more and infinities, and K or Q of 2^60 and more, have no split: a workgroup that meets one starts its
-// part again with the fp32 matrix instructions on the inputs themselves (plain_part), so that infinities go through the
-// arithmetic of the plain fp32 product. A NaN splits into two or three and needs no path of its own.
+// Q and K of 2^60 and more, V of 2^70 and more and infinities are not split: a workgroup that meets one starts its part
+// again with the fp32 matrix instructions on the same tiles in fp32, so that overflow and infinities go through the
+// arithmetic of the plain fp32 product. A NaN splits into NaNs and needs no path of its own.
 //
-// 1000 queries x 8192 keys x 16 heads of 64, against attn_f32_mfma on the same box: 176 us, 424; 2-norm error against
-// fp64 3.6e-7, 8.6e-7; largest error 4.9e-6 of the rms, 8.2e-6.
+// 1000 queries x 8192 keys x 16 heads of 64, N(0, 1), against attn_f32_mfma on the same box: 190 us (177 TFLOP/s), 418;
+// 2-norm error against fp64 3.6e-7, 8.8e-7. Where one channel decides the scores 4.9e-7 against 5.9e-7, with Q five times
+// as large 6.1e-7 against 1.3e-6; a part that starts again, 336 us. Q and K as fp16 pairs under powers of two, 22 bits
+// in half the products, took 160 us, but 7.2e-7 with one channel: not kept. The MFMAs of a tile and wave take 1632
+// cycles and its 350 vector instructions 1400; one barrier per tile holds the two waves of a SIMD in the same phase, so
+// little of the one runs under the other.
 //
 // The key range is cut into parts (attn_f32_plan) where the query tiles alone leave CUs idle: each part writes its
 // maxima, sums and unnormalized output, and attn_f32_combine merges them.
@@ -40,25 +38,19 @@ constexpr int kTile = 32;       // keys per tile
 constexpr int kVP = kTile + 8;  // elements per d row of a V plane (80 bytes: conflict-free 16-byte reads)
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-constexpr float kSplitLimit = 1152921504606846976.0f;  // 2^60
-constexpr float kScaledMin = 512.0f, kScaledMax = 65000.0f;
+// Q and K of 2^60 and more are not split: below, no product leaves fp32's range, and what bf16 has no bits for under
+// 2^-126 is below 2^-60 in a score.
+constexpr float kSplitLimit = 1152921504606846976.0f;
+// The products kept besides hh: hl, lh, mm, hm, mh (lm, ml and ll are at most 2^-25 of a product).
+constexpr int kSmall[5][2] = {{0, 2}, {2, 0}, {1, 1}, {0, 1}, {1, 0}};
 // A lane's 16 probabilities 2^(score - maximum) of a tile sum to less than 2^kSumBits (to at most 16 where the maximum
 // is the largest).
 constexpr int kSumBits = 5;
 // V is held times 2^24, so the lowest part of every normal value is one too; from 2^70 on it is not split (o stays
 // below 2^94 times the number of keys and 2^kSumBits).
 constexpr float kVScale = 16777216.0f, kVUnit = 1.0f / kVScale, kVLimit = 1180591620717411303424.0f;
-
-// Two values as fp16 pairs h, l.
-__device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& l) {
-    const f16x2 hv = __builtin_convertvector((f32x2{a, b}), f16x2);
-    const float ra = fmaf((float)hv.x, -1.0f, a), rb = fmaf((float)hv.y, -1.0f, b);
-    h = __builtin_bit_cast(uint32_t, hv);
-    l = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{ra, rb}), f16x2));
-}
 
 // Two values as bf16 triples h, m, l: 8 bits each, all 24 bits of an fp32 value between them (down to 2^-109).
 __device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
@@ -73,19 +65,6 @@ __device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& 
     l = pack(ra - low(m), rb - high(m));
 }
 
-// 2^e as fp32, e within [-126, 127]
-__device__ __forceinline__ float pow2(int e) { return __builtin_bit_cast(float, (uint32_t)(127 + e) << 23); }
-
-// The exponent that takes a largest magnitude to [2^13, 2^14): 0 for 0, infinities and NaN, at most 74 (magnitudes
-// below 2^-61 keep fewer bits: their products are below 2^-100).
-__device__ __forceinline__ int scale_exp(float mx) {
-    const int e = 13 + 127 - (int)(__builtin_bit_cast(uint32_t, mx) >> 23);
-    return mx > 0.0f && mx < INFINITY ? (e < 74 ? e : 74) : 0;
-}
-
-__device__ __forceinline__ f32x16 mfma(f16x8 a, f16x8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
 __device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
@@ -101,10 +80,9 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
     constexpr int DB = HD / 32;   // 32-wide d blocks of the output
     constexpr int EV = kTile * HD / (64 * NW);  // staged values per thread of K and of V
     constexpr int KP = HD + 8;    // elements per key row of a K plane (conflict-free 16-byte reads)
-    __shared__ __attribute__((aligned(16))) uint16_t k_lds[2][2][kTile * KP];
+    __shared__ __attribute__((aligned(16))) uint16_t k_lds[2][3][kTile * KP];
     __shared__ __attribute__((aligned(16))) uint16_t v_lds[2][3][HD * kVP];
-    __shared__ uint32_t vote[2][NW];
-    __shared__ float key_unit[kTile];  // what the scores of a key place are in units of
+    __shared__ uint32_t beyond[2];  // the tile has values that are not split (never taken back)
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, half = lane >> 5;
@@ -128,38 +106,21 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
     const float* kbase = static_cast<const float*>(p.k) + b * p.kv_bs + h * HD;
     const float* vbase = static_cast<const float*>(p.v) + b * p.kv_bs + h * HD;
 
-    // Q^T operand planes: the lane's query, d = 16 c + 8 half + e, times the query's 2^qe
-    f16x8 qf[2][DC];
-    float qmax = 0.0f;
-    {
+    // the lane's half of its query: x[8 c + e] is d = 16 c + 8 half + e
+    float x[HH];
+    auto load_query = [&]() __attribute__((always_inline)) {
         const float* qrow = qbase + (qi < lq ? qi : lq - 1) * p.ldq;
-        float x[HH];
 #pragma unroll
         for (int i = 0; i < HH; i += 4) {
             const f32x4 a = *reinterpret_cast<const f32x4*>(qrow + 16 * (i >> 3) + 8 * half + (i & 4));
             x[i] = a[0], x[i + 1] = a[1], x[i + 2] = a[2], x[i + 3] = a[3];
-            qmax = fmaxf(qmax, fmaxf(fmaxf(fabsf(a[0]), fabsf(a[1])), fmaxf(fabsf(a[2]), fabsf(a[3]))));
         }
-        qmax = fmaxf(qmax, __shfl_xor(qmax, 32));
-        const float qs = pow2(scale_exp(qmax));
-#pragma unroll
-        for (int c = 0; c < DC; ++c) {
-            uint32_t w[2][4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) split2(x[8 * c + 2 * e] * qs, x[8 * c + 2 * e + 1] * qs, w[0][e], w[1][e]);
-#pragma unroll
-            for (int pl = 0; pl < 2; ++pl)
-                qf[pl][c] = __builtin_bit_cast(f16x8, make_uint4(w[pl][0], w[pl][1], w[pl][2], w[pl][3]));
-        }
-    }
-    // a score's factor to the base-2 domain is cq times its key's unit: ck for the 16 the lane holds
-    const float cq = p.scale_log2 * pow2(-scale_exp(qmax));
+    };
+    load_query();
 
     const int64_t tiles = (lk + kTile - 1) / kTile;
     const int64_t t0 = part * per, t1 = t0 + per < tiles ? t0 + per : tiles;
     float mc = -INFINITY, l_part = 0.0f;  // the running maximum (base-2 domain) and this lane's half of the sum
-    int ke = 0;  // the exponent of the scale of the thread's key of K
-    float ck[16];
     f32x16 o[DB], small[DB];  // the sums of the products hh, and of the others
 #pragma unroll
     for (int t = 0; t < DB; ++t)
@@ -210,10 +171,28 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
             }
         }
     };
-    // votes: 1 K beyond its scale's range, 2 some K within it, 4 some K not 0; 64 a value without a split (K of 2^60
-    // or more, V of kVLimit or more; big: one of the wave's queries)
-    auto stage_tile = [&](int buf, bool big) __attribute__((always_inline)) {
-        const float ks = pow2(ke);
+    if (t0 < t1) load_tile(t0);
+
+    bf16x8 qf[3][DC];  // Q^T operand planes
+    float qmax = 0.0f;
+#pragma unroll
+    for (int c = 0; c < DC; ++c) {
+        uint32_t w[3][4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float a = x[8 * c + 2 * e], b = x[8 * c + 2 * e + 1];
+            split3(a, b, w[0][e], w[1][e], w[2][e]);
+            qmax = fmaxf(qmax, fmaxf(fabsf(a), fabsf(b)));
+        }
+#pragma unroll
+        for (int pl = 0; pl < 3; ++pl)
+            qf[pl][c] = __builtin_bit_cast(bf16x8, make_uint4(w[pl][0], w[pl][1], w[pl][2], w[pl][3]));
+    }
+    if (tid < 2) beyond[tid] = 0;
+    __syncthreads();
+    if (!(qmax < kSplitLimit)) beyond[0] = 1;
+
+    auto stage_tile = [&](int buf) __attribute__((always_inline)) {
         float kmax = 0.0f, vmax = 0.0f;
         uint32_t w[3][EV / 2];
         auto store = [&](uint16_t* dst, int pl) __attribute__((always_inline)) {
@@ -226,12 +205,11 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
         };
 #pragma unroll
         for (int e = 0; e < EV / 2; ++e) {
-            const float x = kr[2 * e] * ks, y = kr[2 * e + 1] * ks;
-            split2(x, y, w[0][e], w[1][e]);
-            kmax = fmaxf(kmax, fmaxf(fabsf(x), fabsf(y)));
+            split3(kr[2 * e], kr[2 * e + 1], w[0][e], w[1][e], w[2][e]);
+            kmax = fmaxf(kmax, fmaxf(fabsf(kr[2 * e]), fabsf(kr[2 * e + 1])));
         }
-        store(&k_lds[buf][0][skey * KP + sd], 0);
-        store(&k_lds[buf][1][skey * KP + sd], 1);
+#pragma unroll
+        for (int pl = 0; pl < 3; ++pl) store(&k_lds[buf][pl][skey * KP + sd], pl);
 #pragma unroll
         for (int e = 0; e < EV / 2; ++e) {
             split3(vr[2 * e] * kVScale, vr[2 * e + 1] * kVScale, w[0][e], w[1][e], w[2][e]);
@@ -239,29 +217,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
         }
 #pragma unroll
         for (int pl = 0; pl < 3; ++pl) store(&v_lds[buf][pl][vd * kVP + vplace], pl);
-        auto any = [&](bool c) __attribute__((always_inline)) { return __builtin_amdgcn_ballot_w64(c) != 0; };
-        uint32_t bits = any(kmax >= kScaledMin) ? 2u : 0u;  // every lane takes part
-        bits |= any(kmax > kScaledMax) ? 1u : 0u;
-        bits |= any(kmax > 0.0f) ? 4u : 0u;
-        bits |= any(big || kmax * pow2(-ke) >= kSplitLimit || vmax >= kVLimit) ? 64u : 0u;
-        if (lane == 0) vote[buf][wave] = bits;
-    };
-    // New scales from the largest finite magnitudes of the keys in kr, and the tile staged into buffer buf with them.
-    // Every wave takes part.
-    auto rescale_tile = [&](int buf, bool big) __attribute__((always_inline)) {
-        auto finite = [](float x) __attribute__((always_inline)) { return fabsf(x) < INFINITY ? fabsf(x) : 0.0f; };
-        float km = 0.0f;
-#pragma unroll
-        for (int i = 0; i < EV; ++i) km = fmaxf(km, finite(kr[i]));
-#pragma unroll
-        for (int off = 1; off < HD / EV; off <<= 1) km = fmaxf(km, __shfl_xor(km, off));
-        ke = scale_exp(km);
-        if (sd == 0) key_unit[skey] = pow2(-ke);
-        __syncthreads();  // the units are in place, and every wave has read the votes that stage_tile writes again
-#pragma unroll
-        for (int r = 0; r < 16; ++r) ck[r] = cq * key_unit[8 * (r >> 2) + 4 * half + (r & 3)];
-        stage_tile(buf, big);
-        __syncthreads();  // the planes and votes are in place, the units have been read
+        if (!(kmax < kSplitLimit && vmax < kVLimit)) beyond[buf] = 1;
     };
 
     // MASK: the last tile, with fewer than 32 keys; FIRST: the part's first tile, whose largest score sets the maximum
@@ -270,19 +226,19 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
         f32x16 s;
 #pragma unroll
         for (int r = 0; r < 16; ++r) s[r] = 0.0f;
-        f16x8 kf[2][DC];
+        bf16x8 kf[3][DC];
 #pragma unroll
-        for (int pl = 0; pl < 2; ++pl)
+        for (int pl = 0; pl < 3; ++pl)
 #pragma unroll
-            for (int c4 = 0; c4 < DC; ++c4)
-                kf[pl][c4] = *reinterpret_cast<const f16x8*>(&k_lds[buf][pl][col * KP + 16 * c4 + 8 * half]);
+            for (int c = 0; c < DC; ++c)
+                kf[pl][c] = *reinterpret_cast<const bf16x8*>(&k_lds[buf][pl][col * KP + 16 * c + 8 * half]);
 #pragma unroll
-        for (int c4 = 0; c4 < DC; ++c4) s = mfma(kf[0][c4], qf[1][c4], s);
+        for (int i = 0; i < 5; ++i)
 #pragma unroll
-        for (int c4 = 0; c4 < DC; ++c4) s = mfma(kf[1][c4], qf[0][c4], s);
+            for (int c = 0; c < DC; ++c) s = mfma(kf[kSmall[i][0]][c], qf[kSmall[i][1]][c], s);
 #pragma unroll
-        for (int c4 = 0; c4 < DC; ++c4) s = mfma(kf[0][c4], qf[0][c4], s);
-        // keys past lk have no score: decided on the scaled scores, since a unit (ck) of tiny operands may be 0
+        for (int c = 0; c < DC; ++c) s = mfma(kf[0][c], qf[0][c], s);
+        // keys past lk have no score
         const int valid = MASK ? (int)(lk - k0) : kTile;
         auto scored = [&](int r, float x) __attribute__((always_inline)) {
             return MASK && 8 * (r >> 2) + 4 * half + (r & 3) >= valid ? -INFINITY : x;
@@ -293,12 +249,12 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
         if (FIRST) {
             float mx = -INFINITY;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, scored(r, s[r] * ck[r]));
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, scored(r, s[r] * p.scale_log2));
             mc = fmaxf(mx, __shfl_xor(mx, 32));
         }
         const float sub = mc == -INFINITY ? 0.0f : mc;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = scored(r, fmaf(s[r], ck[r], -sub));
+        for (int r = 0; r < 16; ++r) s[r] = scored(r, fmaf(s[r], p.scale_log2, -sub));
         f32x16 pr;
         float lt;
         auto probabilities = [&]() __attribute__((always_inline)) {
@@ -348,8 +304,6 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
                 for (int pl = 0; pl < 3; ++pl)
                     vf[t][pl] = *reinterpret_cast<const bf16x8*>(
                         &v_lds[buf][pl][(t * 32 + col) * kVP + 16 * kc + 8 * half]);
-            // hl, lh, mm, hm, mh (lm, ml and ll, at most 2^-25 of a product, are dropped), and hh
-            constexpr int kSmall[5][2] = {{0, 2}, {2, 0}, {1, 1}, {0, 1}, {1, 0}};
 #pragma unroll
             for (int i = 0; i < 5; ++i)
 #pragma unroll
@@ -359,77 +313,23 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
         }
     };
 
-    // The part with fp32 matrix instructions on operands read from memory; the wave on its own, no LDS.
-    auto plain_part = [&]() __attribute__((always_inline)) {
-        const float* qrow = qbase + (qi < lq ? qi : lq - 1) * p.ldq;
-        mc = -INFINITY, l_part = 0.0f;
-#pragma unroll
-        for (int t = 0; t < DB; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) o[t][r] = 0.0f;
-#pragma unroll 1
-        for (int64_t t = t0; t < t1; ++t) {
-            const int64_t k0 = t * kTile;
-            const float* krow = kbase + (k0 + col < lk ? k0 + col : lk - 1) * ldkv;
-            f32x16 s;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = 0.0f;
-#pragma unroll 1
-            for (int i = half * HH; i < half * HH + HH; ++i)
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(krow[i], qrow[i], s, 0, 0, 0);
-            float mx = -INFINITY;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                s[r] = k0 + 8 * (r >> 2) + 4 * half + (r & 3) < lk ? s[r] * p.scale_log2 : -INFINITY;
-                mx = fmaxf(mx, s[r]);
-            }
-            const float m_new = fmaxf(mc, fmaxf(mx, __shfl_xor(mx, 32)));
-            const float sub = m_new == -INFINITY ? 0.0f : m_new;  // every score so far -inf: no weight
-            const float alpha = __builtin_amdgcn_exp2f(mc - sub);
-            mc = m_new;
-            l_part *= alpha;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                s[r] = __builtin_amdgcn_exp2f(s[r] - sub);
-                l_part += s[r];
-            }
-#pragma unroll
-            for (int d = 0; d < DB; ++d)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int64_t key = k0 + 8 * (r >> 2) + 4 * half + (r & 3);
-#pragma unroll
-                for (int d = 0; d < DB; ++d)
-                    o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(key < lk ? vbase[key * ldkv + d * 32 + col] : 0.0f, s[r],
-                                                                o[d], 0, 0, 0);
-            }
-        }
-    };
-
-    if (t0 < t1) load_tile(t0);
-    if (t0 < t1) rescale_tile(0, qmax >= kSplitLimit);
+    // tile t (in buffer buf): the next tile's loads, the product, the next tile's staging and the barrier that publishes
+    // it; false where the tile has values that are not split
     int buf = 0;
     bool plain = false;  // uniform over the workgroup
-    // tile t (in buffer buf): its scales checked, the next tile's loads, the product, the next tile's staging and the
-    // barrier that publishes it; false where the part has to start again
     auto step = [&](int64_t t, auto mask_tag, auto first_tag) __attribute__((always_inline)) {
-        uint32_t votes = 0;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) votes |= vote[buf][w];
-        votes = __builtin_amdgcn_readfirstlane(votes);
-        if (votes & 64u) return false;
-        if ((votes & 1u) || (votes & 6u) == 4u) rescale_tile(buf, false);
+        const uint32_t out = beyond[buf];  // written before the last barrier, and next after this step's
         if (t + 1 < t1) load_tile(t + 1);
         if (active) compute(buf, t * kTile, mask_tag, first_tag);
-        if (t + 1 < t1) stage_tile(buf ^ 1, false);
+        if (t + 1 < t1) stage_tile(buf ^ 1);
         __syncthreads();
         buf ^= 1;
-        return true;
+        return __builtin_amdgcn_readfirstlane(out) == 0;
     };
     const int64_t full = t1 * kTile <= lk ? t1 : t1 - 1;  // the last tile of all may hold fewer keys
     if (t0 < t1) {
+        stage_tile(0);
+        __syncthreads();
         if (full > t0)
             plain = !step(t0, std::false_type{}, std::true_type{});
         else
@@ -437,14 +337,92 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
         for (int64_t t = t0 + 1; t < full && !plain; ++t) plain = !step(t, std::false_type{}, std::false_type{});
         if (full < t1 && full > t0 && !plain) plain = !step(full, std::true_type{}, std::false_type{});
     }
+
+    // The part with fp32 matrix instructions on the values themselves: tiles of fp32 in the same buffers, K [key][d], V
+    // transposed as above. A lane half's 8 values of d or of keys are an instruction's two depths with the other's.
+    constexpr int KF = HD + 4, VF = kTile + 4;  // floats per row (conflict-free 16-byte reads)
+    static_assert(kTile * KF * 4 <= sizeof(k_lds[0]) && HD * VF * 4 <= sizeof(v_lds[0]), "the tiles fit");
+    auto k_f32 = [&](int b) __attribute__((always_inline)) { return reinterpret_cast<float*>(k_lds[b][0]); };
+    auto v_f32 = [&](int b) __attribute__((always_inline)) { return reinterpret_cast<float*>(v_lds[b][0]); };
+    auto stage_plain = [&](int b) __attribute__((always_inline)) {
+        auto store = [&](float* dst, const float (&v)[EV]) __attribute__((always_inline)) {
+            if constexpr (EV == 2)
+                *reinterpret_cast<f32x2*>(dst) = f32x2{v[0], v[1]};
+            else
+#pragma unroll
+                for (int i = 0; i < EV; i += 4)
+                    *reinterpret_cast<f32x4*>(dst + i) = f32x4{v[i], v[i + 1], v[i + 2], v[i + 3]};
+        };
+        store(k_f32(b) + skey * KF + sd, kr);
+        store(v_f32(b) + vd * VF + vplace, vr);
+    };
+    auto compute_plain = [&](int b, int64_t k0) __attribute__((always_inline)) {
+        f32x16 s;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < HH; i += 4) {
+            const f32x4 k4 = *reinterpret_cast<const f32x4*>(k_f32(b) + col * KF + 16 * (i >> 3) + 8 * half + (i & 4));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4[e], x[i + e], s, 0, 0, 0);
+        }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            s[r] = k0 + 8 * (r >> 2) + 4 * half + (r & 3) < lk ? s[r] * p.scale_log2 : -INFINITY;
+            mx = fmaxf(mx, s[r]);
+        }
+        const float m_new = fmaxf(mc, fmaxf(mx, __shfl_xor(mx, 32)));
+        const float sub = m_new == -INFINITY ? 0.0f : m_new;  // every score so far -inf: no weight
+        const float alpha = __builtin_amdgcn_exp2f(mc - sub);
+        mc = m_new;
+        l_part *= alpha;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            s[r] = __builtin_amdgcn_exp2f(s[r] - sub);
+            l_part += s[r];
+        }
+#pragma unroll
+        for (int d = 0; d < DB; ++d)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
+#pragma unroll
+        for (int r = 0; r < 16; r += 4)
+#pragma unroll
+            for (int d = 0; d < DB; ++d) {
+                const f32x4 v4 = *reinterpret_cast<const f32x4*>(v_f32(b) + (d * 32 + col) * VF + 16 * (r >> 3) +
+                                                                 8 * half + (r & 4));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(v4[e], s[r + e], o[d], 0, 0, 0);
+            }
+    };
     // the factor that takes a sum of weights to weights of at most 1, and the maximum those refer to
-    float w = pow2(-kSumBits);
+    float w = 1.0f / (1 << kSumBits);
     mc += (float)kSumBits;
 #pragma unroll
     for (int t = 0; t < DB; ++t) o[t] += small[t];
-    if (plain) {
+    if (plain) {  // (after a barrier: no wave reads the buffers any more)
         w = 1.0f;
-        if (active) plain_part();
+        mc = -INFINITY, l_part = 0.0f;
+#pragma unroll
+        for (int t = 0; t < DB; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[t][r] = 0.0f;
+        load_query();
+        if (t0 < t1) {
+            load_tile(t0);
+            stage_plain(0);
+        }
+        __syncthreads();
+        buf = 0;
+#pragma unroll 1
+        for (int64_t t = t0; t < t1; ++t) {
+            if (t + 1 < t1) load_tile(t + 1);
+            if (active) compute_plain(buf, t * kTile);
+            if (t + 1 < t1) stage_plain(buf ^ 1);
+            __syncthreads();
+            buf ^= 1;
+        }
     }
     const float unit = plain ? 1.0f : kVUnit;  // of o
 

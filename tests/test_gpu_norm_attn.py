@@ -419,9 +419,9 @@ def _attention64(q, k, v, heads, hd):
                                                (257, 2049, 4, 2), (40, 8192, 8, 1), (1000, 1500, 16, 1),
                                                (1700, 90, 16, 1)])
 def test_attention_fp32_split_operands_match_fp64(hd, lq, lk, heads, batch):
-    # fp32 attention on bf16 triples, with and without a cut key range, groups a multiple of 8 or not: 24-bit operands
-    # and fp32 sums of 64 to 8192 terms against fp64: 2^-24 a rounding, at most lk / 16 + 64 of them in sequence, which
-    # grow like their square root: below 2e-6 at 8192 keys
+    # fp32 attention on bf16 triples (all 24 bits of an operand; the products left out are 2^-25 of one), with and without
+    # a cut key range, groups a multiple of 8 or not, against fp64: fp32 sums of up to 8192 terms, each of at most lk / 16
+    # + 64 roundings of 2^-24 in sequence, which grow like their square root: below 2e-6 at 8192 keys
     rng = np.random.default_rng(lq * 7 + lk + hd)
     dim = heads * hd
     q = rng.normal(0, 1, (batch, lq, dim)).astype(np.float32)
@@ -439,15 +439,16 @@ def test_attention_fp32_split_operands_match_fp64(hd, lq, lk, heads, batch):
 @pytest.mark.parametrize("hd", [32, 64])
 @pytest.mark.parametrize("lk", [40, 2000])
 def test_attention_fp32_split_operands_keep_infinities_and_large_values(hd, lk):
-    # keys masked by -inf in one channel (positive queries there), an infinite and a lowest-value V, scores beyond 2^60
-    # and a NaN: where the plain fp32 product is finite, infinite or NaN, so is this one
+    # keys masked by -inf in one channel (positive queries there), an infinite and a lowest-value V, a query beyond 2^60
+    # (each sends its workgroups to the fp32 instructions) and a NaN (which does not): where the plain fp32 product is
+    # finite, infinite or NaN, so is this one
     rng = np.random.default_rng(lk + hd)
     lq, heads = 150, 8
     dim = heads * hd
     q = rng.normal(0, 1, (lq, dim)).astype(np.float32)
     k = rng.normal(0, 1, (lk, dim)).astype(np.float32)
     v = rng.normal(0, 1, (lk, dim)).astype(np.float32)
-    q[:, 0] = 1.0  # one bf16 value, so its low parts are 0
+    q[:, 0] = 1.0
     k[5, 0], k[lk - 1, 0] = -np.inf, -np.inf  # head 0: two keys without weight
     v[7, hd + 3] = np.inf  # head 1: one infinite output column
     v[9, 2 * hd] = np.finfo(np.float32).min  # head 2: the lowest value, finite times its weight
@@ -478,9 +479,8 @@ def test_attention_fp32_split_operands_keep_infinities_and_large_values(hd, lk):
 
 @pytest.mark.parametrize("hd", [32, 64])
 def test_attention_fp32_split_operands_hold_rows_and_columns_of_any_scale(hd):
-    # keys and columns of V whose magnitudes differ by powers of two up to 2^40 and change along the keys, so the
-    # operands' scales change again and again; zero keys and columns among them: each column of V against fp64 at the
-    # accuracy of equal scales
+    # keys and columns of V whose magnitudes differ by powers of two up to 2^40 and change along the keys; zero keys and
+    # columns among them: each column of V against fp64 at the accuracy of equal scales
     rng = np.random.default_rng(31 + hd)
     lq, lk, heads = 200, 1500, 2
     dim = heads * hd
@@ -516,8 +516,8 @@ def test_attention_fp32_without_a_workspace_takes_the_kernel_that_cuts_keys_insi
     assert norm_rel(out.cpu().numpy(), _attention64(q, k, v, heads, hd)) < 2e-6
 
 
-# lq, heads, lk: a cut key range, and one whose query tiles fill the device
-F32_RANGES = [(200, 2, 1507), (4096, 16, 421)]
+# lq, heads, lk: a cut key range (4 waves, parts of several tiles), and one whose query tiles fill the device (8 waves)
+F32_RANGES = [(200, 16, 1507), (4096, 16, 421)]
 
 
 def _attention_f32_inputs(seed, lq, lk, dim):
@@ -547,16 +547,17 @@ def test_attention_fp32_of_vanishing_scores_masks_the_keys_past_the_end(hd, lq, 
 @pytest.mark.parametrize("hd", [32, 64])
 @pytest.mark.parametrize("lq,heads,lk", F32_RANGES)
 @pytest.mark.parametrize("tile", ["first", "middle", "last"])
-def test_attention_fp32_columns_of_v_beside_large_values_without_weight(hd, lq, heads, lk, tile):
+@pytest.mark.parametrize("large", [(1e4, 1e9, -1e12, 1e20), (1e4, 1e9, -1e12, 1e30)])
+def test_attention_fp32_columns_of_v_beside_large_values_without_weight(hd, lq, heads, lk, tile, large):
     # one key of weight e^-100 (or less) with a large V in some columns: each column keeps the accuracy that its own
     # weighted values have in fp32 (see the tests above), since no operand is held relative to the largest of its column
+    # (1e30: the part's fp32 instructions)
     q, k, v = _attention_f32_inputs(3 * hd + lk, lq, lk, heads * hd)
     key = {"first": 7, "middle": lk // 2, "last": lk - 2}[tile]
     q[:, 0] = 1.0
     k[key] = 0.0
     k[key, 0] = -800.0
-    for d, large in enumerate((1e4, 1e9, -1e12, 1e20, 1e30)):
-        v[key, d] = large
+    v[key, :len(large)] = large
     got, want = _attention_f32_head(q, k, v, heads, hd)
     for d in range(hd):
         assert norm_rel(got[:, d], want[:, d]) < 2e-6, d
@@ -596,3 +597,34 @@ def test_attention_fp32_small_weights_count_beside_a_dominant_key(hd, peak):
     got, want = _attention_f32_head(q, k, v, heads, hd)
     for d in range(hd):
         assert norm_rel(got[:, d], want[:, d]) < 8e-6, d
+
+
+@pytest.mark.parametrize("hd", [32, 64])
+@pytest.mark.parametrize("lq,heads,lk", F32_RANGES)
+@pytest.mark.parametrize("tile", ["first", "middle", "last"])
+@pytest.mark.parametrize("q0,k0", [(1.0, -1e3), (1.0, -1e6), (1.0, -1e8), (1.0, -1e9), (1.0, -1e12), (1.0, -1e30), (0.0, 1e9),
+                                   (0.0, 1e30)])
+def test_attention_fp32_keys_beside_one_with_a_large_channel(hd, lq, heads, lk, tile, q0, k0):
+    # a key masked by a large negative channel, or with one that the queries do not read: the other keys' scores (and
+    # its own, where it is not masked) keep fp32's accuracy
+    q, k, v = _attention_f32_inputs(7 * hd + lk, lq, lk, heads * hd)
+    q[:, 0] = q0
+    k[{"first": 5, "middle": lk // 2, "last": lk - 2}[tile], 0] = k0
+    got, want = _attention_f32_head(q, k, v, heads, hd)
+    assert norm_rel(got, want) < 2e-6
+
+
+@pytest.mark.parametrize("hd", [32, 64])
+@pytest.mark.parametrize("lq,heads,lk", F32_RANGES)
+@pytest.mark.parametrize("scale", [1e-12, 1e-6, 1e-4, 1.0, 1e4, 1e12])
+def test_attention_fp32_keys_of_any_scale_and_zero_keys(hd, lq, heads, lk, scale):
+    # K scaled down and Q up by the same factor, or the other way round, with keys that are 0 in every other tile, and
+    # keys and queries of far smaller magnitude among the others
+    q, k, v = _attention_f32_inputs(11 * hd + lk, lq, lk, heads * hd)
+    q /= np.float32(scale)
+    k *= np.float32(scale)
+    k[((np.arange(lk) // 32) % 2 == 0) & (np.arange(lk) % 32 % 3 == 0)] = 0.0
+    k[::7] *= np.float32(1e-6)
+    q[::5] *= np.float32(1e-5)
+    got, want = _attention_f32_head(q, k, v, heads, hd)
+    assert norm_rel(got, want) < 2e-6
