@@ -230,3 +230,16 @@ def test_panel_to_q8_0_inverts_the_gguf_bridge():
     bad[32:34] = np.array([np.float16(0.25)]).view(np.uint8)  # a minimum that is not -128 * scale
     with pytest.raises(ValueError, match="-128"):
         K.panel_to_q8_0(bad, 70, 1024)
+
+
+@pytest.mark.parametrize("hd", [32, 64])
+def test_fp32_attention_asks_for_no_workspace_where_the_binding_passes_none(hd):
+    # up to F32_WHOLE_KEYS keys the binding does not ask for the workspace of a cut key range: the plan cuts none there
+    # (without the workspace such a call would take another kernel than the plan's); it does cut long ranges of few rows
+    lib = L.load()
+    for lk in range(1, L.F32_WHOLE_KEYS + 1, 31):
+        for heads in list(range(1, 40)) + [64, 85, 128, 256, 500]:
+            for lq in (1, 32, 33, 100, 127, 128, 129, 255, 256, 257, 400, 512, 1000, 4000):
+                assert lib.idolq_attention_f32_workspace(1, lq, lk, heads, hd) == 0, (lq, lk, heads)
+    assert lib.idolq_attention_f32_workspace(1, 40, 8192, 8, hd) > 0
+    assert lib.idolq_attention_f32_workspace(2, 8192, 8192, 16, hd) == 0
