@@ -260,11 +260,13 @@ int launch_tile(GemmParams p, bool w4, hipStream_t stream) {
 
 int launch_i8_rows(const GemmParams& p, bool w4, hipStream_t stream) {
     // Up to 16 rows: the weights are what is read, in 32-row tiles for more of them in flight. From 256 tiles of 128 x
-    // 128 on (a round of the CUs) those: 2048^3 56.7 against 62.7 us with 64 x 64, 4096^3 347 against 400; below,
-    // 64 x 64: 2000 x 1024 x 1024 (128 tiles) 23.3 against 34.5.
+    // 128 on (a round of the CUs) those, but for shallow depths, where their epilogue and the few stages of the one
+    // workgroup a CU holds leave it waiting: k of 64, 1300 x 5586 32.1 us against 26.0 with 64 x 64; 1024, 4096^2 123
+    // against 119; 1536, 160 against 162; 2048^3 59 against 63, 4096^3 347 against 389. Below 256 tiles 64 x 64: 2000 x
+    // 1024 x 1024 (128 tiles) 23.3 against 34.5.
     if (p.m <= 16) return launch_tile<16, 32, 2, 1>(p, w4, stream);
     const int64_t large = (int64_t)((p.m + 127) / 128) * ((p.n + 127) / 128);
-    if (large >= 256) return launch_tile<128, 128, 8, 4>(p, w4, stream);
+    if (large >= 256 && p.k > 1024) return launch_tile<128, 128, 8, 4>(p, w4, stream);
     return launch_tile<64, 64, 8, 4>(p, w4, stream);
 }
 

@@ -113,7 +113,7 @@ def test_dequant_writes_every_block(n, k):
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 33, 32), (16, 64, 160), (17, 63, 128), (65, 129, 224), (130, 64, 4096),
-                                   (2049, 2050, 96), (1, 4096, 256)])
+                                   (2049, 2050, 96), (1, 4096, 256), (2049, 2050, 1056), (2050, 2047, 1088)])
 @pytest.mark.parametrize("skew", [0, 2])
 def test_int8_row_major_tiles_fold_block_by_block(m, n, k, skew):
     # every tile of the row-major INT8 kernel (16 x 32, 64 x 64, 128 x 128), partial tiles, a last stage of 1 to 3
@@ -632,3 +632,17 @@ def test_block_dots_past_two_to_the_32_bytes_of_codes():
     want = np.einsum("mbe,nbe->mnb", tail.reshape(64, k // 32, 32).astype(np.int32), codes)
     assert np.array_equal(dots[m - 64:].cpu().numpy(), want)
     assert not dots[:m - 64].any()
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 33, 64), (65, 129, 128), (1000, 130, 128), (65, 129, 192)])
+def test_exact_of_shallow_depths_takes_the_tile_kernel(m, n, k):
+    # up to two pairs of blocks the aligned rows take the 64 x 64 tile that rows off 16 bytes take at any depth (the split
+    # kernel is slower there): the same bits; from three pairs on the order of the sums differs (6 terms: below 1e-6)
+    rng = np.random.default_rng(m + n + k)
+    a, w = rng.normal(0, 1, (m, k + 1)).astype(np.float32), to_dev(q8(rng, n, k, 0.05))
+    off = L.gemm(to_dev(a)[:, 1:], w, n, mode=L.MODE_EXACT)
+    on = L.gemm(to_dev(np.ascontiguousarray(a[:, 1:])), w, n, mode=L.MODE_EXACT)
+    if k <= 128:
+        assert torch.equal(on, off)
+    else:
+        assert norm_rel(on.cpu().numpy(), off.cpu().numpy()) < 1e-6
