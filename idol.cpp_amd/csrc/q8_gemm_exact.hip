@@ -6,9 +6,11 @@
 // unchanged, and each wave takes its operands out of them in registers (alignbyte for the blocks that start two bytes
 // past a dword, a byte conversion and half a pack per code), so nothing waits for a second trip through LDS. Loads are
 // issued two stages ahead into registers; a full stage's carry no masks. At 1024 rows a CU has one workgroup, and what
-// bounds it is the chain of a stage (LDS round trip, conversion, MFMAs, fold): four blocks a stage for the 64 x 64
-// tile, two for the larger, whose LDS holds no more. Against the kernel this replaced, which converted the weights to
-// bf16 in LDS: 1024 x 4096 x 1024 41.5 -> 36 us, 8192 x 2048 x 1024 147 -> 125, 1024 x 1024 x 1024 20 -> 15.5.
+// bounds it is the chain of a stage (LDS round trip, conversion, MFMAs, fold): two blocks a stage, or four for 64 x 64
+// tiles of deep products (launch_exact_rows); the larger tiles' LDS holds no more than two. Against the kernel this
+// replaced, which converted the weights to bf16 in LDS: 1024 x 4096 x 1024 40 -> 36 us, 8192 x 2048 x 1024 157 -> 134,
+// 310 x 5572 x 512 18.1 -> 14.6.
+#include "q8_dma.h"
 #include "q8_epilogue.h"
 
 namespace idolq {
@@ -223,9 +225,9 @@ __global__ __launch_bounds__(512, 2) void q8_gemm_exact_kernel(GemmParams p) {
 
 // A 64 x 64 tile whose eight waves each take every eighth pair of blocks for the whole tile: each converted code and
 // each x operand feeds twice the products of a 32 x 32 wave tile, and a wave stages its pair in LDS of its own, so the
-// loop has no barrier; the waves' sums meet in LDS at the end, in wave order. Where choose_tile takes 64 x 64: 1024 x
-// 1024 x 4096 47 -> 38 us against the kernel above, 1024 x 1024 x 1024 15.5 -> 15; 1024 x 4096 x 1024, four rounds of
-// such tiles, 54 against 36 with 128 x 128. Vector work (conversion, split, fold: about 430 instructions per pair and
+// loop has no barrier; the waves' sums meet in LDS at the end, in wave order. 1024 x 1024 x 4096 37 us against 43 with the
+// kernel above, 1024 x 1024 x 1024 14.2 against 15.5; 1024 x 4096 x 1024, four rounds of such tiles, 52 against 36 with
+// 128 x 128. Vector work (conversion, split, fold: about 430 instructions per pair and
 // wave) and the MFMAs bound it, little of the one under the other.
 __global__ __launch_bounds__(512, 2) void q8_gemm_exact_split_kernel(GemmParams p) {
     constexpr int kTileMN = 64, kWaves = 8;
@@ -415,13 +417,23 @@ int launch_split(GemmParams p, hipStream_t stream) {
 }  // namespace
 
 int launch_exact_rows(const GemmParams& p, bool w4, hipStream_t stream) {
+    // Measured with each tile over 23 shapes at depths of 256, 1024 and 4096, the choice is within 2% of the best. At
+    // 1024 x 1024 x 1024 the split kernel takes 14.2 us, 128 x 64 21.5; at 1024 x 1280 x 1024, past one round of 64 x 64
+    // tiles, 24.3 against 21.7; at 1024 x 3072 x 1024 128 x 64 takes 39.8, 128 x 128 32.8.
     static const TileChoice cands[] = {{128, 128, 1.0f}, {128, 64, 1.0f}, {64, 64, 0.75f}};
     const TileChoice t = choose_tile(p.m, p.n, cands, 3);
     if (t.bn == 128) return launch_tile<128, 128, 2>(p, w4, stream);
     if (t.bm == 128) return launch_tile<128, 64, 2>(p, w4, stream);
-    // the split kernel: aligned rows of whole pairs of blocks, 64 rows of x below 2^31 bytes
-    if (w4 && p.x_aligned && p.ldx < 1 << 23) return launch_split(p, stream);
-    return launch_tile<64, 64, 4>(p, w4, stream);
+    // 64 x 64, measured in us as split kernel / four blocks a stage / two. Two leave room for two workgroups a CU and take
+    // the fewest bytes of a short row: best up to a depth of 512 in one round of the CUs (1000 x 1024 x 64 8.1 / 7.0 / 6.3,
+    // x 512 10.8 / 10.6 / 10.8, x 1024 13.7 / 14.7 / 15.4), up to 2048 in more (310 x 5572 x 64 13.9 / 11.8 / 7.4, x 1024
+    // 24.4 / 26.6 / 21.7, x 2048 37.6 / 43.5 / 37.5, x 4096 62.8 / 76.7 / 66.5). Beyond, the split kernel for aligned rows
+    // of whole pairs of blocks, 64 rows of x below 2^31 bytes.
+    const bool one_round = (int64_t)((p.m + 63) / 64) * ((p.n + 63) / 64) <= cu_count();
+    const bool shallow = p.k <= (one_round ? 512 : 2048);
+    if (!shallow && w4 && p.x_aligned && p.ldx < 1 << 23) return launch_split(p, stream);
+    if (!shallow && one_round) return launch_tile<64, 64, 4>(p, w4, stream);
+    return launch_tile<64, 64, 2>(p, w4, stream);
 }
 
 }  // namespace idolq

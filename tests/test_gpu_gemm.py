@@ -634,15 +634,14 @@ def test_block_dots_past_two_to_the_32_bytes_of_codes():
     assert not dots[:m - 64].any()
 
 
-@pytest.mark.parametrize("m,n,k", [(17, 33, 64), (65, 129, 128), (1000, 130, 128), (65, 129, 192)])
+@pytest.mark.parametrize("m,n,k", [(17, 33, 64), (65, 129, 192), (1000, 130, 512), (65, 129, 576), (33, 16390, 576)])
 def test_exact_of_shallow_depths_takes_the_tile_kernel(m, n, k):
-    # up to two pairs of blocks the aligned rows take the 64 x 64 tile that rows off 16 bytes take at any depth (the split
-    # kernel is slower there): the same bits; from three pairs on the order of the sums differs (6 terms: below 1e-6)
+    # up to a depth of 512, or where 64 x 64 tiles fill more than a round of the CUs, aligned rows take the tile that rows
+    # off 16 bytes take at any depth (the split kernel is slower there): the same bits; a deeper product in one round is
+    # split, and the order of its sums differs (18 terms: below 1e-6)
     rng = np.random.default_rng(m + n + k)
     a, w = rng.normal(0, 1, (m, k + 1)).astype(np.float32), to_dev(q8(rng, n, k, 0.05))
     off = L.gemm(to_dev(a)[:, 1:], w, n, mode=L.MODE_EXACT)
     on = L.gemm(to_dev(np.ascontiguousarray(a[:, 1:])), w, n, mode=L.MODE_EXACT)
-    if k <= 128:
-        assert torch.equal(on, off)
-    else:
-        assert norm_rel(on.cpu().numpy(), off.cpu().numpy()) < 1e-6
+    assert torch.equal(on, off) == ((m, n, k) != (65, 129, 576))
+    assert norm_rel(on.cpu().numpy(), off.cpu().numpy()) < 1e-6
