@@ -536,18 +536,19 @@ __device__ __forceinline__ void wide_tiles(const GemmParams& p, const WideSplit&
         const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(p.y, 0, 0x7fffffff, kRaw);
         const __amdgpu_buffer_rsrc_t rr =
             __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.res ? p.res : p.y), 0, p.res ? 0x7fffffff : 0, kRaw);
-        // the bias is fp32 or T: a buffer for each, the other one of no bytes, whose loads read the 0 that is added
+        // the bias is fp32 or T: 16 bytes at four fp32 values, or at eight T of which four are used (past the end: 0)
         const bool b32 = p.bias_dt == IDOLQ_F32;
-        const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.bias ? p.bias : p.y), 0,
-                                                                            p.bias && b32 ? 0x7fffffff : 0, kRaw);
-        const __amdgpu_buffer_rsrc_t rbt = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.bias ? p.bias : p.y), 0,
-                                                                             p.bias && !b32 ? 0x7fffffff : 0, kRaw);
+        const uint32_t bsz = b32 ? 4 : 2;
+        const __amdgpu_buffer_rsrc_t rb =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.bias ? p.bias : p.y), 0, p.bias ? (uint32_t)p.n * bsz : 0, kRaw);
         auto bias4 = [&](int c0, bool ok) __attribute__((always_inline)) {
-            const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, ok ? (uint32_t)c0 * 4 : kOff, 0, 0));
-            const auto w = __builtin_amdgcn_raw_buffer_load_b64(rbt, ok ? (uint32_t)c0 * 2 : kOff, 0, 0);
+            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+            const u32x4 w = __builtin_bit_cast(
+                u32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, ok ? c0 * bsz : kOff, 0, 0));
             const f32x2 lo = __builtin_convertvector(__builtin_bit_cast(T2, (uint32_t)w[0]), f32x2);
             const f32x2 hi = __builtin_convertvector(__builtin_bit_cast(T2, (uint32_t)w[1]), f32x2);
-            return f32x4{v[0] + lo.x, v[1] + lo.y, v[2] + hi.x, v[3] + hi.y};
+            const f32x4 v = __builtin_bit_cast(f32x4, w);
+            return f32x4{b32 ? v[0] : lo.x, b32 ? v[1] : lo.y, b32 ? v[2] : hi.x, b32 ? v[3] : hi.y};
         };
         const f32x4 b = bias4(col, col_ok);
         f32x4 bacc[CT][4];  // !RES: the biases in the accumulator layout (stage_chunk_act)
