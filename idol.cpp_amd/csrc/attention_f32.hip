@@ -510,20 +510,22 @@ __global__ __launch_bounds__(256) void attn_f32_combine(AttnParams p, int parts,
 
 // The cheapest of the kernel's forms (waves per workgroup), numbers of parts and, with waves 0, attn_f32_mfma, from
 // measured times in microseconds: a tile step of the 4-wave form alone on its CU and of two there, of the 8-wave form with
-// one wave of a SIMD at work (up to 128 queries) and with both; one and a half steps to start, and the merge (a launch and
-// the partials written and read back). attn_f32_mfma steps 32 keys in each of its 4 waves, and each round of its
-// workgroups starts anew. At 16 heads of 64, the form taken against the next: 300 queries x 64 keys attn_f32_mfma 6.8 us,
-// 4 waves 8.6; 736 x 181 4 waves 16.3, parts of two 18.8, attn_f32_mfma 20.2; 128 x 700 8 waves in 11 parts 15.2, 4 waves
-// in 22 18.2, attn_f32_mfma 22.3; 1000 x 8192 8 waves in 4 parts 176, 4 waves 195; 4096 x 421 8 waves 44.3, 4 waves 48.4.
+// one wave of a SIMD at work (up to 128 queries) and with both; the steps' worth of a workgroup's start and end, and the
+// merge (a launch and the partials written and read back). attn_f32_mfma steps 32 keys in each of its 4 waves, and each
+// round of its workgroups starts anew. At 16 heads of 64, the form taken against the next: 100 queries x 64 keys
+// attn_f32_mfma 6.5 us, 4 waves 7.9; 1000 x 128 4 waves 12.2, attn_f32_mfma 14.5; 736 x 181 4 waves 16.3, parts of two
+// 18.8, attn_f32_mfma 20.2; 128 x 700 8 waves in 11 parts 15.2, 4 waves in 22 18.2, attn_f32_mfma 22.3; 1000 x 8192 8
+// waves in 4 parts 176, 4 waves 195; 4096 x 421 8 waves 44.3, 4 waves 48.4.
 AttnF32Plan attn_f32_plan(int64_t batch, int64_t lq, int64_t lk, int64_t heads, int64_t head_dim) {
     struct Steps {
-        double mfma, mfma_start, alone, two, half, both;
+        double mfma, mfma_start, mfma_first, alone, two, half, both;  // mfma_first: less for the first round's start
     };
-    constexpr Steps kSteps64{2.85, 2.5, 1.7, 2.75, 1.45, 2.45}, kSteps32{1.65, 1.5, 1.08, 1.56, 1.0, 1.5};
+    constexpr Steps kSteps64{2.85, 2.9, 1.8, 1.7, 2.75, 1.45, 2.45}, kSteps32{1.65, 0.7, 0.0, 1.08, 1.56, 1.0, 1.5};
     const Steps& c = head_dim == 64 ? kSteps64 : kSteps32;
     const int64_t cus = cu_count(), tiles = (lk + kTile - 1) / kTile;
     AttnF32Plan best{0, 1};
-    double best_cost = (((lq + 31) / 32 * heads * batch + cus - 1) / cus) * ((tiles + 3) / 4 * c.mfma + c.mfma_start);
+    double best_cost =
+        (((lq + 31) / 32 * heads * batch + cus - 1) / cus) * ((tiles + 3) / 4 * c.mfma + c.mfma_start) - c.mfma_first;
     for (int nw = 4; nw <= 8; nw += 4) {
         const int64_t base = (lq + 32 * nw - 1) / (32 * nw) * heads * batch, slots = nw == 4 ? 2 * cus : cus;
         for (int s = 1; s <= 64 && s <= tiles && (s == 1 || s * base <= slots); ++s) {
@@ -531,7 +533,7 @@ AttnF32Plan attn_f32_plan(int64_t batch, int64_t lq, int64_t lk, int64_t heads, 
             if (s > 1 && (tiles + per - 1) / per != s) continue;  // every part has tiles
             const double step = nw == 8 ? (lq <= 128 ? c.half : c.both) : wgs <= cus ? c.alone : c.two;
             const double merge = s == 1 ? 0.0 : 4.0 + 2.5e-6 * head_dim * (s * batch * heads * lq);
-            const double cost = (per + 1.5) * step * ((wgs + slots - 1) / slots) + merge;
+            const double cost = (per + (nw == 8 ? 1.9 : 1.5)) * step * ((wgs + slots - 1) / slots) + merge;
             if (cost < best_cost) best = {nw, s}, best_cost = cost;
         }
     }
