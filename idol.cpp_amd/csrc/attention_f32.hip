@@ -3,27 +3,27 @@
 // The fp32 matrix instructions (v_mfma_f32_32x32x2_f32) take 64 cycles for the products the bf16 ones do in 4, so an
 // fp32 product made of six bf16 products has 2.7 times the rate. h = bf16(x), m = bf16(x - h) and l = bf16(x - h - m)
 // hold all 24 bits of x at its own exponent: no operand has a scale, and none loses bits to a larger one beside it (a
-// key may carry 1e12 in one channel, V 1e30 at a key of no weight, a query's weights may fall to 1e-30). Of the nine
+// key may carry 1e12 in one channel, V 1e20 at a key of no weight, a query's weights may fall to 1e-30). Of the nine
 // products hh, hm, mh, mm, hl and lh are kept; lm, ml and ll are at most 2^-25 of one. Everything is accumulated in
 // fp32, hh of the product with V in an accumulator of its own: it rounds once per 16 keys where the fp32 instruction
-// rounds after 2, so the result's error is no larger than that kernel's (below).
+// rounds after 2, so the result's 2-norm error is no larger than that kernel's (below).
 //
 // attn_f32_split<HD, NW>: a workgroup of NW waves owns 32 NW queries of one (batch, head) and a range of 32-key tiles.
-// The tile's K and V are split once per workgroup on their way into LDS (K planes [key][d], V planes transposed [d][key],
-// the keys of a 16-chunk in the order in which a lane of the score accumulator holds them), two tile buffers, one barrier
-// per tile. Scores are computed transposed, S^T = K Q^T, so a lane holds 16 scores of one query and its probabilities,
-// split in registers, are the B operand of O^T = V^T P^T.
+// The tile's K and V are split once per workgroup on their way into LDS (K planes [key][d], V planes transposed
+// [d][key], the keys of a 16-chunk in the order in which a lane of the score accumulator holds them), two tile buffers,
+// one barrier per tile. Scores are computed transposed, S^T = K Q^T, so a lane holds 16 scores of one query and its
+// probabilities, split in registers, are the B operand of O^T = V^T P^T.
 //
 // Q and K of 2^60 and more, V of 2^70 and more and infinities are not split: a workgroup that meets one starts its part
 // again with the fp32 matrix instructions on the same tiles in fp32, so that overflow and infinities go through the
 // arithmetic of the plain fp32 product. A NaN splits into NaNs and needs no path of its own.
 //
-// 1000 queries x 8192 keys x 16 heads of 64, N(0, 1), against attn_f32_mfma on the same box: 190 us (177 TFLOP/s), 418;
-// 2-norm error against fp64 3.6e-7, 8.8e-7. Where one channel decides the scores 4.9e-7 against 5.9e-7, with Q five times
-// as large 6.1e-7 against 1.3e-6; a part that starts again, 336 us. Q and K as fp16 pairs under powers of two, 22 bits
-// in half the products, took 160 us, but 7.2e-7 with one channel: not kept. The MFMAs of a tile and wave take 1632
-// cycles and its 350 vector instructions 1400; one barrier per tile holds the two waves of a SIMD in the same phase, so
-// little of the one runs under the other.
+// 1000 queries x 8192 keys x 16 heads of 64, N(0, 1), against attn_f32_mfma on the same box: 188 us (179 TFLOP/s), 411;
+// 2-norm error against fp64 3.6e-7, 8.8e-7. Where one channel decides the scores 4.9e-7 against 5.9e-7, with Q five
+// times as large 6.1e-7 against 1.3e-6. With an infinite V, parts that start again: 332 us against 366. Q and K as fp16
+// pairs under powers of two, 22 bits in half the products, took 160 us, but 7.2e-7 with one channel: not kept. Counters
+// of that call: MFMA busy 197 k and vector instructions 151 k of 327 k cycles a SIMD, waves waiting 29% of their time:
+// little of the one runs under the other (the barrier of every tile holds the two waves of a SIMD in the same phase).
 //
 // The key range is cut into parts (attn_f32_plan) where the query tiles alone leave CUs idle: each part writes its
 // maxima, sums and unnormalized output, and attn_f32_combine merges them.
@@ -127,9 +127,9 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[t][r] = 0.0f, small[t][r] = 0.0f;
 
-    // Staging. K: thread t takes EV values of a key, a row to HD / EV consecutive threads. V: thread t takes d row t % HD
-    // and EV keys whose places in that row of the plane are contiguous: place 16 kc + 8 half + e holds key 16 kc +
-    // 8 (e / 4) + 4 half + e % 4.
+    // Staging. K: thread t takes EV values of a key, a row to HD / EV consecutive threads. V: thread t takes d row
+    // t % HD and EV keys whose places in that row of the plane are contiguous: place 16 kc + 8 half + e holds key
+    // 16 kc + 8 (e / 4) + 4 half + e % 4.
     const int skey = tid / (HD / EV), sd = EV * (tid % (HD / EV));
     const int vd = tid % HD, vplace = tid / HD * EV;
     const int vkey = (vplace >> 4) * 16 + ((vplace >> 2) & 1) * 8 + ((vplace >> 3) & 1) * 4 + (vplace & 3);
@@ -313,8 +313,8 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
         }
     };
 
-    // tile t (in buffer buf): the next tile's loads, the product, the next tile's staging and the barrier that publishes
-    // it; false where the tile has values that are not split
+    // tile t (in buffer buf): the next tile's loads, the product, the next tile's staging and the barrier that
+    // publishes it; false where the tile has values that are not split
     int buf = 0;
     bool plain = false;  // uniform over the workgroup
     auto step = [&](int64_t t, auto mask_tag, auto first_tag) __attribute__((always_inline)) {
@@ -509,13 +509,13 @@ __global__ __launch_bounds__(256) void attn_f32_combine(AttnParams p, int parts,
 }  // namespace
 
 // The cheapest of the kernel's forms (waves per workgroup), numbers of parts and, with waves 0, attn_f32_mfma, from
-// measured times in microseconds: a tile step of the 4-wave form alone on its CU and of two there, of the 8-wave form with
-// one wave of a SIMD at work (up to 128 queries) and with both; the steps' worth of a workgroup's start and end, and the
-// merge (a launch and the partials written and read back). attn_f32_mfma steps 32 keys in each of its 4 waves, and each
-// round of its workgroups starts anew. At 16 heads of 64, the form taken against the next: 100 queries x 64 keys
-// attn_f32_mfma 6.5 us, 4 waves 7.9; 1000 x 128 4 waves 12.2, attn_f32_mfma 14.5; 736 x 181 4 waves 16.3, parts of two
-// 18.8, attn_f32_mfma 20.2; 128 x 700 8 waves in 11 parts 15.2, 4 waves in 22 18.2, attn_f32_mfma 22.3; 1000 x 8192 8
-// waves in 4 parts 176, 4 waves 195; 4096 x 421 8 waves 44.3, 4 waves 48.4.
+// measured times in microseconds: a tile step of the 4-wave form alone on its CU and of two there, of the 8-wave form
+// with one wave of a SIMD at work (up to 128 queries) and with both; the steps' worth of a workgroup's start and end,
+// and the merge (a launch and the partials written and read back). attn_f32_mfma steps 32 keys in each of its 4 waves,
+// and each round of its workgroups starts anew. At heads of 64, the form taken against the next: 12 heads, 100 queries
+// x 64 keys attn_f32_mfma 6.5 us, 4 waves 7.9; 16 heads, 1000 x 128 4 waves 12.2, attn_f32_mfma 14.5; 736 x 181 4 waves
+// 16.3, parts of two 18.8, attn_f32_mfma 20.2; 128 x 700 8 waves in 11 parts 15.2, 4 waves in 22 18.2, attn_f32_mfma
+// 22.3; 1000 x 8192 8 waves in 4 parts 176, 4 waves 195; 4096 x 421 8 waves 44.3, 4 waves 48.4.
 AttnF32Plan attn_f32_plan(int64_t batch, int64_t lq, int64_t lk, int64_t heads, int64_t head_dim) {
     struct Steps {
         double mfma, mfma_start, mfma_first, alone, two, half, both;  // mfma_first: less for the first round's start
