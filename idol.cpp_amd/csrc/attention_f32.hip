@@ -6,7 +6,9 @@
 // key may carry 1e12 in one channel, V 1e20 at a key of no weight, a query's weights may fall to 1e-30). Of the nine
 // products hh, hm, mh, mm, hl and lh are kept; lm, ml and ll are at most 2^-25 of one. Everything is accumulated in
 // fp32, hh of the product with V in an accumulator of its own: it rounds once per 16 keys where the fp32 instruction
-// rounds after 2, so the result's 2-norm error is no larger than that kernel's (below).
+// rounds after 2, so the result's 2-norm error is no larger than that kernel's (below). Q is scaled (log2(e) /
+// sqrt(head_dim), one rounding, where that kernel rounds the scaled scores) before it is split: the maximum is then one
+// of the scores and not another rounding of it, which at scores beyond 2^31 would differ by more than an exponent holds.
 //
 // attn_f32_split<HD, NW>: a workgroup of NW waves owns 32 NW queries of one (batch, head) and a range of 32-key tiles.
 // The tile's K and V are split once per workgroup on their way into LDS (K planes [key][d], V planes transposed
@@ -18,11 +20,11 @@
 // again with the fp32 matrix instructions on the same tiles in fp32, so that overflow and infinities go through the
 // arithmetic of the plain fp32 product. A NaN splits into NaNs and needs no path of its own.
 //
-// 1000 queries x 8192 keys x 16 heads of 64, N(0, 1), against attn_f32_mfma on the same box: 188 us (179 TFLOP/s), 411;
-// 2-norm error against fp64 3.6e-7, 8.8e-7. Where one channel decides the scores 4.9e-7 against 5.9e-7, with Q five
-// times as large 6.1e-7 against 1.3e-6. With an infinite V, parts that start again: 332 us against 366. Q and K as fp16
+// 1000 queries x 8192 keys x 16 heads of 64, N(0, 1), against attn_f32_mfma on the same box: 185 us (181 TFLOP/s), 415;
+// 2-norm error against fp64 3.3e-7, 8.8e-7. Where one channel decides the scores 4.0e-7 against 5.9e-7, with Q five
+// times as large 5.0e-7 against 1.3e-6. With an infinite V, parts that start again: 333 us against 392. Q and K as fp16
 // pairs under powers of two, 22 bits in half the products, took 160 us, but 7.2e-7 with one channel: not kept. Counters
-// of that call: MFMA busy 197 k and vector instructions 151 k of 327 k cycles a SIMD, waves waiting 29% of their time:
+// of that call: MFMA busy 197 k and vector instructions 151 k of 320 k cycles a SIMD, waves waiting 27% of their time:
 // little of the one runs under the other (the barrier of every tile holds the two waves of a SIMD in the same phase).
 //
 // The key range is cut into parts (attn_f32_plan) where the query tiles alone leave CUs idle: each part writes its
@@ -173,7 +175,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
     };
     if (t0 < t1) load_tile(t0);
 
-    bf16x8 qf[3][DC];  // Q^T operand planes
+    bf16x8 qf[3][DC];  // Q^T operand planes, times the scale: scores come in the base-2 domain
     float qmax = 0.0f;
 #pragma unroll
     for (int c = 0; c < DC; ++c) {
@@ -181,7 +183,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const float a = x[8 * c + 2 * e], b = x[8 * c + 2 * e + 1];
-            split3(a, b, w[0][e], w[1][e], w[2][e]);
+            split3(a * p.scale_log2, b * p.scale_log2, w[0][e], w[1][e], w[2][e]);
             qmax = fmaxf(qmax, fmaxf(fabsf(a), fabsf(b)));
         }
 #pragma unroll
@@ -238,53 +240,45 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
             for (int c = 0; c < DC; ++c) s = mfma(kf[kSmall[i][0]][c], qf[kSmall[i][1]][c], s);
 #pragma unroll
         for (int c = 0; c < DC; ++c) s = mfma(kf[0][c], qf[0][c], s);
-        // keys past lk have no score
-        const int valid = MASK ? (int)(lk - k0) : kTile;
-        auto scored = [&](int r, float x) __attribute__((always_inline)) {
-            return MASK && 8 * (r >> 2) + 4 * half + (r & 3) >= valid ? -INFINITY : x;
-        };
+        if (MASK) {
+            const int valid = (int)(lk - k0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (8 * (r >> 2) + 4 * half + (r & 3) >= valid) s[r] = -INFINITY;
+        }
         // The maximum mc is the first tile's, raised only where a lane's probabilities of a tile sum to 2^kSumBits or
         // more, infinity and NaN included: no maximum is taken of the other tiles, the sum is needed anyway (a
-        // wave-uniform branch). While every score was -inf, mc is -inf and 0 is subtracted: no weight.
-        if (FIRST) {
+        // wave-uniform branch). It is one of the scores as they are, so that the largest difference is 0 however large
+        // they are. While every score was -inf, mc is -inf and 0 is subtracted: no weight.
+        auto largest = [&]() __attribute__((always_inline)) {
             float mx = -INFINITY;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, scored(r, s[r] * p.scale_log2));
-            mc = fmaxf(mx, __shfl_xor(mx, 32));
-        }
-        const float sub = mc == -INFINITY ? 0.0f : mc;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = scored(r, fmaf(s[r], p.scale_log2, -sub));
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
+            return fmaxf(mx, __shfl_xor(mx, 32));
+        };
+        if (FIRST) mc = largest();
         f32x16 pr;
         float lt;
         auto probabilities = [&]() __attribute__((always_inline)) {
+            const float sub = mc == -INFINITY ? 0.0f : mc;
             float l2[2] = {0.0f, 0.0f};
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                pr[r] = __builtin_amdgcn_exp2f(s[r]);
+                pr[r] = __builtin_amdgcn_exp2f(s[r] - sub);
                 l2[r & 1] += pr[r];
             }
             lt = l2[0] + l2[1];
         };
         probabilities();
         if (!FIRST && __builtin_amdgcn_ballot_w64(!(lt < (float)(1 << kSumBits)) || mc == -INFINITY) != 0) {
-            float mx = -INFINITY;
+            const float raised = fmaxf(mc, largest());
+            const float alpha = mc < raised ? __builtin_amdgcn_exp2f(mc - raised) : 1.0f;
+            mc = raised;
+            l_part *= alpha;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
-            mx = fmaxf(mx, __shfl_xor(mx, 32));
-            const bool none = mc == -INFINITY;
-            const float delta = none || mx > 0.0f ? mx : 0.0f;
-            if (delta > -INFINITY) {  // else still no score above -inf
-                const float alpha = none ? 0.0f : __builtin_amdgcn_exp2f(-delta);
-                mc = sub + delta;
-                l_part *= alpha;
+            for (int t = 0; t < DB; ++t)
 #pragma unroll
-                for (int t = 0; t < DB; ++t)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) o[t][r] *= alpha, small[t][r] *= alpha;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) s[r] -= delta;
-            }
+                for (int r = 0; r < 16; ++r) o[t][r] *= alpha, small[t][r] *= alpha;
             probabilities();
         }
         l_part += lt;
@@ -396,13 +390,9 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
                 for (int e = 0; e < 4; ++e) o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(v4[e], s[r + e], o[d], 0, 0, 0);
             }
     };
-    // the factor that takes a sum of weights to weights of at most 1, and the maximum those refer to
-    float w = 1.0f / (1 << kSumBits);
-    mc += (float)kSumBits;
 #pragma unroll
     for (int t = 0; t < DB; ++t) o[t] += small[t];
     if (plain) {  // (after a barrier: no wave reads the buffers any more)
-        w = 1.0f;
         mc = -INFINITY, l_part = 0.0f;
 #pragma unroll
         for (int t = 0; t < DB; ++t)
@@ -437,10 +427,10 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f32_split(AttnParams p, int q
                 const int d = t * 32 + 2 * r + 4 * half;
                 f32x4 v;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = o[t][r + e] * w * unit;
+                for (int e = 0; e < 4; ++e) v[e] = o[t][r + e] * unit;
                 *reinterpret_cast<f32x4*>(part_o + row * HD + d) = v;
             }
-        if (half == 0) *reinterpret_cast<f32x2*>(part_ml + 2 * row) = f32x2{mc, l * w};
+        if (half == 0) *reinterpret_cast<f32x2*>(part_ml + 2 * row) = f32x2{mc, l};
         return;
     }
     const float inv = 1.0f / l;

@@ -628,3 +628,24 @@ def test_attention_fp32_keys_of_any_scale_and_zero_keys(hd, lq, heads, lk, scale
     q[::5] *= np.float32(1e-5)
     got, want = _attention_f32_head(q, k, v, heads, hd)
     assert norm_rel(got, want) < 2e-6
+
+
+@pytest.mark.parametrize("hd", [32, 64])
+@pytest.mark.parametrize("lq,heads,lk", F32_RANGES)
+@pytest.mark.parametrize("scale", [1e8, 1e10, 1e15])
+def test_attention_fp32_of_scores_far_beyond_the_exponent(hd, lq, heads, lk, scale):
+    # finite scores of 1e8 and more, growing along the keys: the largest one's weight is 1 whatever its rounding, and
+    # the others, which differ by far more than that rounding, have none
+    q, k, v = _attention_f32_inputs(13 * hd + lk, lq, lk, heads * hd)
+    k *= (scale * (1.0 + np.arange(lk) / lk)[:, None]).astype(np.float32)
+    got, want = _attention_f32_head(q, k, v, heads, hd)
+    assert norm_rel(got, want) < 2e-6
+
+
+@pytest.mark.parametrize("hd", [32, 64])
+def test_attention_fp32_of_one_key_is_its_v(hd):
+    # a single key has weight 1: V itself, bit for bit (enough queries for the split kernel)
+    q, k, v = _attention_f32_inputs(hd, 4000, 1, 16 * hd)
+    out = torch.empty((4000, 16 * hd), device=DEV)
+    L.attention(to_dev(q), to_dev(k), to_dev(v), 1, 4000, 1, 16, hd, 16 * hd, 16 * hd, 0, 0, out, 16 * hd, 0)
+    assert torch.equal(out, to_dev(v).expand_as(out))
