@@ -20,7 +20,7 @@
 // again with the fp32 matrix instructions on the same tiles in fp32, so that overflow and infinities go through the
 // arithmetic of the plain fp32 product. A NaN splits into NaNs and needs no path of its own.
 //
-// 1000 queries x 8192 keys x 16 heads of 64, N(0, 1), against attn_f32_mfma on the same box: 185 us (181 TFLOP/s), 415;
+// 1000 queries x 8192 keys x 16 heads of 64, N(0, 1), against attn_f32_mfma on the same card: 185 us (181 TFLOP/s), 415;
 // 2-norm error against fp64 3.3e-7, 8.8e-7. Where one channel decides the scores 4.0e-7 against 5.9e-7, with Q five
 // times as large 5.0e-7 against 1.3e-6. With an infinite V, parts that start again: 333 us against 392. Q and K as fp16
 // pairs under powers of two, 22 bits in half the products, took 160 us, but 7.2e-7 with one channel: not kept. Counters
